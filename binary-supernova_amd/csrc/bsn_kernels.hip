@@ -284,24 +284,65 @@ __global__ void k_floors(const GridDev* __restrict__ grids, const int64_t* __res
 
 template <typename T> struct Prec;
 template <> struct Prec<double> {
-    template <int DIR>
+    using Carry = ex::WenoCarry;
+    // big: uniform over the wave, set where a stencil holds a value too large
+    // for the flux's shared reciprocals (big_cell) or gamma is out of range
+    template <int DIR, bool WALK = false>
     __device__ static void flux(const double (&c)[4][6], const double (&p)[6], const GridDev& G,
-                                double F[5]) {
-        ex::interface_flux<DIR>(c, p, G.gamma, G.gfac, F);
+                                bool big, double F[5], Carry (&w)[5]) {
+        if (__builtin_expect(!ex::interface_flux_shared<DIR, WALK>(c, p, G.gamma, G.gfac, big, F, w), 0)) {
+            volatile double s[30];
+#pragma unroll
+            for (int m = 0; m < 6; ++m) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) s[6 * q + m] = c[q][m];
+                s[24 + m] = p[m];
+            }
+            ex::interface_flux_plain<DIR>([&](int q, int m) { return s[6 * q + m]; }, G.gamma, G.gfac, F);
+            // the carry is formed again, so that it need not be kept here
+            if (WALK) ex::interface_walk_start<1>(c, p, w);
+        }
+    }
+    // The same where at(q, m) can read the stencil again from LDS.
+    template <int DIR, typename At>
+    __device__ static void flux_at(const double (&c)[4][6], const double (&p)[6], const GridDev& G,
+                                bool big, double F[5], Carry (&w)[5], At&& at) {
+        if (__builtin_expect(!ex::interface_flux_shared<DIR, false>(c, p, G.gamma, G.gfac, big, F, w), 0)) {
+            asm volatile("" ::: "memory");      // at reads again: nothing is kept for it
+            ex::interface_flux_plain<DIR>(at, G.gamma, G.gfac, F);
+        }
+    }
+    __device__ static void start(const double (&c)[4][6], const double (&p)[6], Carry (&w)[5]) {
+        ex::interface_walk_start(c, p, w);
     }
     __device__ static double pressure(const double (&u)[5], double g) {
         return ex::cell_pressure(u[0], u[1], u[2], u[3], u[4], g);
     }
+    __device__ static bool big_cell(const double (&u)[5], double p) {
+        return ex::cell_big(u[0], u[1], u[2], u[3], p);
+    }
+    __device__ static bool big_gamma(double g) { return !ex::gamma_ok(g); }
 };
 template <> struct Prec<float> {
-    template <int DIR>
-    __device__ static void flux(const float (&c)[4][6], const float (&p)[6], const GridDev& G,
-                                float F[5]) {
-        sp::interface_flux<DIR>(c, p, G.gf32[0], G.gf32[1], G.gf32[2], F);
+    using Carry = sp::WenoCarry;
+    template <int DIR, bool WALK = false>
+    __device__ static void flux(const float (&c)[4][6], const float (&p)[6], const GridDev& G, bool,
+                                float F[5], Carry (&w)[5]) {
+        sp::interface_flux<DIR, WALK>(c, p, G.gf32[0], G.gf32[1], G.gf32[2], F, w);
+    }
+    template <int DIR, typename At>
+    __device__ static void flux_at(const float (&c)[4][6], const float (&p)[6], const GridDev& G, bool big,
+                                float F[5], Carry (&w)[5], At&&) {
+        flux<DIR>(c, p, G, big, F, w);
+    }
+    __device__ static void start(const float (&c)[4][6], const float (&p)[6], Carry (&w)[5]) {
+        sp::interface_walk_start(c, p, w);
     }
     __device__ static double pressure(const double (&u)[5], double g) {
         return sp::cell_pressure(u[0], u[1], u[2], u[3], u[4], g);
     }
+    __device__ static bool big_cell(const double (&)[5], double) { return false; }
+    __device__ static bool big_gamma(double) { return false; }
 };
 
 // Stores the flux of interface f along DIR with cross indices ci, cj
@@ -335,12 +376,7 @@ __global__ __launch_bounds__(W * H, (DIR == 0 && W == 64 && H == 4 && sizeof(T) 
     const int tid = threadIdx.x;
     int t0, t1;
     chunk(ntiles, t0, t1);
-    // interface f along DIR with cross indices ci, cj (active, 0-based)
-    auto emit = [&](const GridDev& G, const T (&c)[4][6], const T (&p)[6], int f, int ci, int cj) {
-        T F[5];
-        Prec<T>::template flux<DIR>(c, p, G, F);
-        store_face<DIR>(G, F, f, ci, cj);
-    };
+    typename Prec<T>::Carry nc[5];               // unused: no indicators are carried between tiles
     for (int t = t0; t < t1; ++t) {
         const Tile tl = tiles[t];
         const GridDev& G = grids[tl.g];
@@ -353,6 +389,7 @@ __global__ __launch_bounds__(W * H, (DIR == 0 && W == 64 && H == 4 && sizeof(T) 
             const int ci = tl.b + tid, cj = tl.c;
             const int f = DIR == 0 ? G.nx : DIR == 1 ? G.ny : G.nz;
             if (ci < (DIR == 0 ? G.ny : G.nx)) {
+                bool big = Prec<T>::big_gamma(G.gamma);
 #pragma unroll
                 for (int m = 0; m < 6; ++m) {
                     double u[5];
@@ -360,11 +397,14 @@ __global__ __launch_bounds__(W * H, (DIR == 0 && W == 64 && H == 4 && sizeof(T) 
                     else if (DIR == 1) load_cell<1, true, FAST>(G, NG + ci, f + m, NG + cj, u);
                     else               load_cell<2, true, FAST>(G, NG + ci, NG + cj, f + m, u);
                     const double pr = Prec<T>::pressure(u, G.gamma);
+                    big |= Prec<T>::big_cell(u, pr);
 #pragma unroll
                     for (int q = 0; q < 4; ++q) c[q][m] = (T)u[q];
                     p[m] = (T)pr;
                 }
-                emit(G, c, p, f, ci, cj);
+                T F[5];
+                Prec<T>::template flux<DIR>(c, p, G, __ballot(big) != 0, F, nc);
+                store_face<DIR>(G, F, f, ci, cj);
             }
             continue;
         }
@@ -384,6 +424,7 @@ __global__ __launch_bounds__(W * H, (DIR == 0 && W == 64 && H == 4 && sizeof(T) 
             const double* rowU = G.U + uidx(G, 0, pjb, pk);
             const uint32_t roff = (uint32_t)((pj - pjb) * G.pitch) * 8u;
             double u[2][5];
+            bool big = Prec<T>::big_gamma(G.gamma);
 #pragma unroll
             for (int r = 0; r < 2; ++r) {
                 int pi = min(tl.a + (r ? W + min(x, 4) : x), Nx - 1);
@@ -398,6 +439,7 @@ __global__ __launch_bounds__(W * H, (DIR == 0 && W == 64 && H == 4 && sizeof(T) 
                     if ((G.lmode & 2) && pi >= NG && pi < NG + G.nx)
                         apply_floor<FAST>(u[r], G.rho_floor, G.P_floor, G.gamma);
                     const double pr = Prec<T>::pressure(u[r], G.gamma);
+                    big |= Prec<T>::big_cell(u[r], pr);
 #pragma unroll
                     for (int q = 0; q < 4; ++q) lds[q][h][b] = (T)u[r][q];
                     lds[4][h][b] = (T)pr;
@@ -409,6 +451,7 @@ __global__ __launch_bounds__(W * H, (DIR == 0 && W == 64 && H == 4 && sizeof(T) 
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
             __builtin_amdgcn_wave_barrier();
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            const bool wbig = __ballot(big) != 0;        // any cell of the wave's rows
             const int f = tl.a + x, ci = tl.b + h;
             if (f < G.nx && ci < G.ny) {
 #pragma unroll
@@ -418,7 +461,8 @@ __global__ __launch_bounds__(W * H, (DIR == 0 && W == 64 && H == 4 && sizeof(T) 
                     p[m] = lds[4][h][x + m];
                 }
                 T F[5];
-                Prec<T>::template flux<0>(c, p, G, F);
+                Prec<T>::template flux_at<0>(c, p, G, wbig, F, nc,
+                                             [&](int q, int m) { return lds[q][h][x + m]; });
                 T* rowF = (T*)G.F[0] + ((int64_t)tl.c * G.ny + tl.b + hb) * G.fp[0];
                 const uint32_t fo = (uint32_t)((h - hb) * G.fp[0] + f) * (uint32_t)sizeof(T);
 #pragma unroll
@@ -432,6 +476,7 @@ __global__ __launch_bounds__(W * H, (DIR == 0 && W == 64 && H == 4 && sizeof(T) 
             continue;
         }
         // stage cells into LDS
+        bool big = Prec<T>::big_gamma(G.gamma);
         for (int e = tid; e < SA * SB; e += NT) {
             const int a = e / SB, b = e - a * SB;
             int pi, pj, pk;
@@ -450,12 +495,15 @@ __global__ __launch_bounds__(W * H, (DIR == 0 && W == 64 && H == 4 && sizeof(T) 
                 double u[5];
                 load_cell<DIR, true, FAST>(G, pi, pj, pk, u);
                 const double pr = Prec<T>::pressure(u, G.gamma);
+                big |= Prec<T>::big_cell(u, pr);
 #pragma unroll
                 for (int q = 0; q < 4; ++q) lds[q][a][b] = (T)u[q];
                 lds[4][a][b] = (T)pr;
             }
         }
-        __syncthreads();
+        // any cell of the tile (the FP64 form asks; the barrier orders the LDS)
+        if constexpr (FAST) __syncthreads();
+        else                big = __syncthreads_or(big);
         const int x = tid % W, h = tid / W;
         int f, ci;
         bool valid;
@@ -474,7 +522,11 @@ __global__ __launch_bounds__(W * H, (DIR == 0 && W == 64 && H == 4 && sizeof(T) 
                     c[q][m] = DIR == 0 ? lds[q][h][x + m] : lds[q][h + m][x];
                 p[m] = DIR == 0 ? lds[4][h][x + m] : lds[4][h + m][x];
             }
-            emit(G, c, p, f, ci, tl.c);
+            T F[5];
+            Prec<T>::template flux_at<DIR>(c, p, G, big, F, nc, [&](int q, int m) {
+                return DIR == 0 ? lds[q][h][x + m] : lds[q][h + m][x];
+            });
+            store_face<DIR>(G, F, f, ci, tl.c);
         }
         __syncthreads();
     }
@@ -503,6 +555,7 @@ __global__ __launch_bounds__(256) void k_fxwalk(const GridDev* __restrict__ grid
     __shared__ T lds[5][4][SB];
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     auto at = [](int b) { return b + (b >> 2); };
+    typename Prec<T>::Carry nw[5];               // of the edge tiles, which carry nothing
     int t0, t1;
     chunk(ntiles, t0, t1);
     for (int t = t0; t < t1; ++t) {
@@ -515,23 +568,26 @@ __global__ __launch_bounds__(256) void k_fxwalk(const GridDev* __restrict__ grid
             if (r < G.ny * G.nz) {
                 const int jr = r % G.ny, kr = r / G.ny;
                 T c[4][6], p[6];
+                bool big = Prec<T>::big_gamma(G.gamma);
 #pragma unroll
                 for (int m = 0; m < 6; ++m) {
                     double u[5];
                     load_cell<0, true, FAST>(G, G.nx + m, NG + jr, NG + kr, u);
                     const double pr = Prec<T>::pressure(u, G.gamma);
+                    big |= Prec<T>::big_cell(u, pr);
 #pragma unroll
                     for (int q = 0; q < 4; ++q) c[q][m] = (T)u[q];
                     p[m] = (T)pr;
                 }
                 T F[5];
-                Prec<T>::template flux<0>(c, p, G, F);
+                Prec<T>::template flux<0>(c, p, G, __ballot(big) != 0, F, nw);
                 store_face<0>(G, F, G.nx, jr, kr);
             }
             continue;
         }
         const int f0 = tl.a, j0 = tl.b, k = tl.c & ZT_K0_MASK, n = tl.c >> ZT_LEN_SHIFT;
         const int nc = n + 5;
+        bool big = Prec<T>::big_gamma(G.gamma);
         {
             // every thread issues all of its loads before it uses the first
             // (indices clamped into the grid, so the loads need no branch),
@@ -553,13 +609,16 @@ __global__ __launch_bounds__(256) void k_fxwalk(const GridDev* __restrict__ grid
                     if ((G.lmode & 2) && f0 + b >= NG && f0 + b < NG + G.nx)
                         apply_floor<FAST>(u[r], G.rho_floor, G.P_floor, G.gamma);
                     const double pr = Prec<T>::pressure(u[r], G.gamma);
+                    big |= Prec<T>::big_cell(u[r], pr);
 #pragma unroll
                     for (int q = 0; q < 4; ++q) lds[q][a][at(b)] = (T)u[r][q];
                     lds[4][a][at(b)] = (T)pr;
                 }
             }
         }
-        __syncthreads();
+        // any cell of the tile (the FP64 form asks; the barrier orders the LDS)
+        if constexpr (FAST) __syncthreads();
+        else                big = __syncthreads_or(big);
         const int j = j0 + w;
         const int b0 = (lane * n) >> 6, len = (((lane + 1) * n) >> 6) - b0;
         T Fb[OUT ? KMAX : 1][5];
@@ -572,14 +631,11 @@ __global__ __launch_bounds__(256) void k_fxwalk(const GridDev* __restrict__ grid
             };
 #pragma unroll
             for (int m = 0; m < 5; ++m) place(m, b0 + m);
-            sp::WenoCarry wc[5];
-            if constexpr (FAST) sp::interface_walk_start(c, p, wc);
+            typename Prec<T>::Carry wc[5];
+            if constexpr (FAST) Prec<T>::start(c, p, wc);
             auto step = [&](int m, T (&F)[5]) {
                 place(5, b0 + m + 5);
-                if constexpr (FAST)
-                    sp::interface_flux<0, true>(c, p, G.gf32[0], G.gf32[1], G.gf32[2], F, wc);
-                else
-                    Prec<T>::template flux<0>(c, p, G, F);
+                Prec<T>::template flux<0, FAST>(c, p, G, big, F, wc);
 #pragma unroll
                 for (int s = 0; s < 5; ++s) {
 #pragma unroll
@@ -638,8 +694,10 @@ __global__ __launch_bounds__(256) void k_fxwalk(const GridDev* __restrict__ grid
 // cell per interface straight from HBM (lanes along x: coalesced), and the
 // split form carries the smoothness indicators that consecutive interfaces
 // share.  A run of len interfaces reads len + 5 cells.
+// The FP64 form carries them too, with their reciprocals, at 255 VGPRs, 2 waves
+// per SIMD.
 template <int DIR, typename T>
-__global__ __launch_bounds__(256, sizeof(T) == 4 ? 4 : 1) void k_fwalk(const GridDev* __restrict__ grids,
+__global__ __launch_bounds__(256, sizeof(T) == 4 ? 4 : 2) void k_fwalk(const GridDev* __restrict__ grids,
                                                const Tile* __restrict__ tiles, int ntiles) {
     constexpr bool FAST = sizeof(T) == 4;        // split form
     int t0, t1;
@@ -664,6 +722,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 4 : 1) void k_fwalk(const Gri
         T c[4][6], p[6];
         double nxt[5];
         int npf = 0;
+        bool big = Prec<T>::big_gamma(G.gamma);
         // cells along the walk are read once (halo cells of neighbouring
         // runs aside): streaming loads.  The load is raw and the floor is
         // applied when the cell is placed, so that the next cell's load stays
@@ -682,6 +741,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 4 : 1) void k_fwalk(const Gri
             if ((G.lmode & 2) && npf >= NG && npf < NG + (DIR == 1 ? G.ny : G.nz))
                 apply_floor<FAST>(nxt, G.rho_floor, G.P_floor, G.gamma);
             const double pr = Prec<T>::pressure(nxt, G.gamma);
+            big |= __ballot(Prec<T>::big_cell(nxt, pr)) != 0;
 #pragma unroll
             for (int q = 0; q < 4; ++q) c[q][slot] = (T)nxt[q];
             p[slot] = (T)pr;
@@ -689,17 +749,14 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 4 : 1) void k_fwalk(const Gri
 #pragma unroll
         for (int m = 0; m < 5; ++m) { fetch(f0 + m); place(m); }
         fetch(f0 + 5);
-        sp::WenoCarry wc[5];
-        if constexpr (FAST) sp::interface_walk_start(c, p, wc);
+        typename Prec<T>::Carry wc[5];
+        Prec<T>::start(c, p, wc);
         const int fend = f0 + len;
         auto step = [&](int f) {
             place(5);                                   // cell f+5 (padded)
             if (f + 1 < fend) fetch(f + 6);             // in flight during the flux
             T F[5];
-            if constexpr (FAST)
-                sp::interface_flux<DIR, true>(c, p, G.gf32[0], G.gf32[1], G.gf32[2], F, wc);
-            else
-                Prec<T>::template flux<DIR>(c, p, G, F);
+            Prec<T>::template flux<DIR, true>(c, p, G, big, F, wc);
             // store_face's layout, from the wave's first row
             T* fb = (T*)G.F[DIR] + (DIR == 1 ? ((int64_t)cc0 * (G.ny + 1) + f) * G.fp[1]
                                              : ((int64_t)f * G.ny + cc0) * G.fp[2]);
@@ -995,6 +1052,9 @@ __global__ __launch_bounds__(256, WB) void k_zupdate(const GridDev* __restrict__
                                                      const Tile* __restrict__ tiles, int ntiles,
                                                      int stage, int do_cfl) {
     constexpr bool FAST = sizeof(T) == 4;        // split form
+    // the FP64 carry (60 VGPRs) does not fit beside the update's operands in 2
+    // waves per SIMD: with it, spilled, the 192^3 step took 5.52 ms against 5.34
+    constexpr bool CARRY = FAST;
     __shared__ double ring[RING ? 4 : 1][5][RING ? 256 : 1];
     const int rt = RING ? (int)threadIdx.x : 0;
     int t0, t1;
@@ -1021,6 +1081,7 @@ __global__ __launch_bounds__(256, WB) void k_zupdate(const GridDev* __restrict__
             const uint32_t fyo = (uint32_t)(j * G.fp[1] + i) * (uint32_t)sizeof(T);
             double nxt[5];
             int npz = 0;
+            bool big = Prec<T>::big_gamma(G.gamma);
             // the z window and the base state are read once per launch:
             // streaming loads (2.7 % on this kernel at 256^3 against cached
             // loads; the x and y fluxes, whose faces neighbouring lanes and
@@ -1046,6 +1107,7 @@ __global__ __launch_bounds__(256, WB) void k_zupdate(const GridDev* __restrict__
                         apply_floor<FAST>(nxt, G.rho_floor, G.P_floor, G.gamma);
                 }
                 const double pr = Prec<T>::pressure(nxt, G.gamma);
+                big |= __ballot(Prec<T>::big_cell(nxt, pr)) != 0;
 #pragma unroll
                 for (int q = 0; q < 4; ++q) c[q][slot] = (T)nxt[q];
                 p[slot] = (T)pr;
@@ -1085,8 +1147,8 @@ __global__ __launch_bounds__(256, WB) void k_zupdate(const GridDev* __restrict__
             fetch(k0 + 5);
             // split form: the smoothness indicators that consecutive
             // interfaces share are carried along the column
-            sp::WenoCarry wc[5];
-            if constexpr (FAST) sp::interface_walk_start(c, p, wc);
+            typename Prec<T>::Carry wc[5];
+            if constexpr (CARRY) Prec<T>::start(c, p, wc);
             T fz0[5];                                   // the previous interface's z flux
             for (int f = k0; f <= kend; ++f) {
                 place(5);                               // cell f+5
@@ -1094,10 +1156,7 @@ __global__ __launch_bounds__(256, WB) void k_zupdate(const GridDev* __restrict__
                 const int k = f - 1;                    // the cell finished in this iteration
                 if (PF == 1 && f > k0) operands(k);
                 T F[5];
-                if constexpr (FAST)
-                    sp::interface_flux<2, true>(c, p, G.gf32[0], G.gf32[1], G.gf32[2], F, wc);
-                else
-                    Prec<T>::template flux<2>(c, p, G, F);
+                Prec<T>::template flux<2, CARRY>(c, p, G, big, F, wc);
                 if (G.nzkeep > 0) {
                     // an interface the flux registers read: store it as the
                     // z-flux sweep would (adjacent tiles both compute their

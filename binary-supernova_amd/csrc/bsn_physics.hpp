@@ -199,22 +199,10 @@ __device__ __forceinline__ void hllc_normal(double rL, double mnL, double mt1L, 
     }
 }
 
-// One interface flux along direction DIR (0 = x, 1 = y, 2 = z) from the
-// six-cell stencil c[q][s] (q = rho, mx, my, mz; s = 0..5 for cells i-2..i+3
-// of the reference's src/gpu_kernels.jl:61-82) and cell pressures p[s].
+// The energies of the face states, then HLLC along DIR.
 template <int DIR>
-__device__ __forceinline__ void interface_flux(const double (&c)[4][6], const double (&p)[6],
-                                               double g, double gfac, double F[5]) {
-    double L[4], R[4];
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-        weno5_pair(c[q][0], c[q][1], c[q][2], c[q][3], c[q][4], c[q][5], L[q], R[q]);
-    double P_maxL = jl_max(jl_max(jl_max(jl_max(p[0], p[1]), p[2]), p[3]), p[4]);
-    double P_maxR = jl_max(jl_max(jl_max(jl_max(p[1], p[2]), p[3]), p[4]), p[5]);
-    double PLw, PRw;
-    weno5_pair(p[0], p[1], p[2], p[3], p[4], p[5], PLw, PRw);
-    double PL = jl_clamp(PLw, 0.0, P_maxL);
-    double PR = jl_clamp(PRw, 0.0, P_maxR);
+__device__ __forceinline__ void hllc_faces(const double (&L)[4], const double (&R)[4], double PL,
+                                           double PR, double g, double gfac, double F[5]) {
     double EL = EL_from_P(PL, L[0], L[1], L[2], L[3], g);
     double ER = EL_from_P(PR, R[0], R[1], R[2], R[3], g);
     double G[5];
@@ -228,6 +216,333 @@ __device__ __forceinline__ void interface_flux(const double (&c)[4][6], const do
         hllc_normal(L[0], L[3], L[1], L[2], EL, R[0], R[3], R[1], R[2], ER, g, gfac, G);
         F[0] = G[0]; F[1] = G[2]; F[2] = G[3]; F[3] = G[1]; F[4] = G[4];
     }
+}
+
+// One interface flux along direction DIR (0 = x, 1 = y, 2 = z), every
+// operation as the reference writes it.  at(q, m) reads the six-cell stencil
+// (q = rho, mx, my, mz, P; m = 0..5 for cells i-2..i+3 of the reference's
+// src/gpu_kernels.jl:61-82) from memory.  The kernels come here rarely, and
+// their waves per SIMD are set by the registers of their largest path: the
+// quantities go through one loop body and their face values through scratch.
+template <int DIR, typename At>
+__device__ __forceinline__ void interface_flux_plain(At&& at, double g, double gfac, double F[5]) {
+    volatile double W[5][2];
+#pragma unroll 1
+    for (int q = 0; q < 5; ++q) {
+        double l, r;
+        weno5_pair(at(q, 0), at(q, 1), at(q, 2), at(q, 3), at(q, 4), at(q, 5), l, r);
+        W[q][0] = l;
+        W[q][1] = r;
+    }
+    const double L[4] = {W[0][0], W[1][0], W[2][0], W[3][0]};
+    const double R[4] = {W[0][1], W[1][1], W[2][1], W[3][1]};
+    double mid = at(4, 1);
+#pragma unroll 1
+    for (int m = 2; m < 5; ++m) mid = jl_max(mid, at(4, m));
+    // the maximum over p[0..4] and over p[1..5] in any order: pressures are
+    // +0 or more, and NaN propagates from every place
+    const double PL = jl_clamp(W[4][0], 0.0, jl_max(at(4, 0), mid));
+    const double PR = jl_clamp(W[4][1], 0.0, jl_max(mid, at(4, 5)));
+    hllc_faces<DIR>(L, R, PL, PR, g, gfac, F);
+}
+
+// ---------------------------------------------------------------------------
+// The same flux with shared reciprocals.
+//
+// An FP64 division a / b compiles to 11 instructions: two scalings, v_rcp_f64
+// (a quarter-rate operation), two Newton steps (4 FMA) to a reciprocal r of b,
+// q = a r, its residual, the corrected quotient q - (b q - a) r and a fix-up
+// (Markstein's scheme).  The scalings and the fix-up act only on operands near
+// the ends of the exponent range, zeros, infinities and NaN.  Where they do
+// nothing the quotient is a function of r, so divisions by one denominator
+// share r: the first costs 8 instructions, each further one 3, and the bits
+// are those of the full division.  WENO5-Z has 12 divisions per quantity by 7
+// distinct denominators; a walk carries the reciprocals of the indicators
+// that consecutive interfaces share, which leaves 5.  HLLC divides 7 times by
+// each side's density.  At 256^3 an FP64 y walk issues 1268 VALU instructions
+// per interface instead of 1949: 1.13 -> 0.79 ms; the tiled x sweep 1.18 ->
+// 0.89 ms, the fused z sweep and update 1.38 -> 1.12 ms, the step 11.4 -> 8.75.
+//
+// Ranges.  interface_flux_shared refuses (the callers then take
+// interface_flux_plain) unless every rho of the stencil is below 2^96 in
+// magnitude, every m and P below 2^180 (or NaN), gamma - 1 is within
+// [2^-40, 2^40] and each face P is at least 2^-600, or zero with every face
+// momentum zero or at least 2^-200.  Then
+//   * indicators are below 2^367 and their denominators eps + beta within
+//     [1e-36, 2^367]; a numerator tau may be tiny, and a quotient that then
+//     rounds differently is below 2^-840: it enters only as 1 + t t, which is
+//     1 either way.  t is below 2^487, the weights' denominators within
+//     [1, 2^976];
+//   * densities are clamped to at least 1e-30, and the energy, pressure and
+//     sound speed terms over a density are zero or at least 2^-850;
+//   * a velocity over a momentum of at least 2^-900 is at least 2^-1000.
+//     Where a wave holds smaller ones, its velocities take full divisions:
+//     ahead of a front the momenta fall through all magnitudes (in a 64^3
+//     Sedov blast up to a third of the waves hold momenta below 2^-900);
+//   * 0.5 |m|^2 may underflow, but where it is below 2^-900 the face P is at
+//     least 2^-600, the kinetic energy below 2^-800, and it is absorbed in
+//     E = P/(gamma-1) + KE and in E - KE.
+// NaN operands give NaN on both paths.
+constexpr double kBigRho = 7.922816251426434e+28;  // 2^96
+constexpr double kBig = 1.532495540865889e+54;     // 2^180
+
+struct Recip { double d, r; };
+
+__device__ __forceinline__ Recip recip(double d) {
+    double r = __builtin_amdgcn_rcp(d);
+    r = __builtin_fma(r, __builtin_fma(-d, r, 1.0), r);
+    r = __builtin_fma(r, __builtin_fma(-d, r, 1.0), r);
+    return {d, r};
+}
+// x / R.d.  The residual is taken as b q - x so that a zero x keeps its sign
+// (b > 0).
+__device__ __forceinline__ double quot(double x, const Recip& R) {
+    const double q = x * R.r;
+    return __builtin_fma(-__builtin_fma(R.d, q, -x), R.r, q);
+}
+
+// max of two values neither of which is -0; a NaN operand is dropped (one
+// instruction; __builtin_fmax first quiets each operand with another)
+__device__ __forceinline__ double hmax(double a, double b) {
+    double r;
+    asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ __forceinline__ double hmaxabs(double a, double b) {
+    double r;
+    asm("v_max_f64 %0, |%1|, |%2|" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+
+// Whether a cell's values rule out the shared reciprocals (NaN does not).
+__device__ __forceinline__ bool cell_big(double r, double mx, double my, double mz, double p) {
+    return fabs(r) >= kBigRho || hmaxabs(hmaxabs(mx, my), hmaxabs(mz, p)) >= kBig;
+}
+__device__ __forceinline__ bool gamma_ok(double g) {
+    return g - 1.0 >= 0x1p-40 && g - 1.0 <= 0x1p40;
+}
+
+// An indicator with the reciprocal of its WENO-Z denominator.
+struct Ind { double b, r; };
+
+// 13/12 s^2 + 1/4 t^2: the product with 1/4 is exact, so the fused sum rounds
+// as the reference's two operations do.
+__device__ __forceinline__ Ind indicator(double s, double t) {
+    const double b = __builtin_fma(1.0 / 4.0, t * t, (13.0 / 12.0) * (s * s));
+    return {b, recip(1e-36 + b).r};
+}
+// x - 2y + z, x - 4y + 3z and 3x - 4y + z: products with 2 and 4 are exact
+__device__ __forceinline__ double d2(double x, double y, double z) { return __builtin_fma(-2.0, y, x) + z; }
+__device__ __forceinline__ double dA(double x, double y, double z) { return __builtin_fma(-4.0, y, x) + 3.0 * z; }
+__device__ __forceinline__ double dC(double x, double y, double z) { return __builtin_fma(-4.0, y, 3.0 * x) + z; }
+
+__device__ __forceinline__ double wenoz_mix(const Ind& i0, const Ind& i1, const Ind& i2, double d0,
+                                            double d1, double d2_, double q0, double q1, double q2) {
+    const double tau5 = fabs(i0.b - i2.b);
+    const double t0 = quot(tau5, {1e-36 + i0.b, i0.r});
+    const double t1 = quot(tau5, {1e-36 + i1.b, i1.r});
+    const double t2 = quot(tau5, {1e-36 + i2.b, i2.r});
+    const double a0 = d0 * (1.0 + t0 * t0);
+    const double a1 = d1 * (1.0 + t1 * t1);
+    const double a2 = d2_ * (1.0 + t2 * t2);
+    const Recip S = recip(a0 + a1 + a2);
+    return quot(a0, S) * q0 + quot(a1, S) * q1 + quot(a2, S) * q2;
+}
+
+// What a walk carries per quantity: the indicators of positions 0 and 1 (the
+// one-sided form right beta1 took at them two and one interfaces ago, which is
+// left beta0) and left beta2 of position 2 (right beta2 of the last interface).
+struct WenoCarry { Ind A0, A1, C2; };
+
+__device__ __forceinline__ void weno5_walk_start(double a0, double a1, double a2, double a3,
+                                                 double a4, WenoCarry& w) {
+    w.A0 = indicator(d2(a0, a1, a2), dA(a0, a1, a2));
+    w.A1 = indicator(d2(a1, a2, a3), dA(a1, a2, a3));
+    w.C2 = indicator(d2(a2, a3, a4), dC(a2, a3, a4));
+}
+
+template <bool WALK>
+__device__ __forceinline__ void weno5_pair_shared(double a0, double a1, double a2, double a3,
+                                                  double a4, double a5, WenoCarry& w, double& vl,
+                                                  double& vr) {
+    const double qL0 = (1.0 / 3.0) * a0 + (-7.0 / 6.0) * a1 + (11.0 / 6.0) * a2;
+    const double qC  = (-1.0 / 6.0) * a1 + (5.0 / 6.0) * a2 + (1.0 / 3.0) * a3;
+    const double qR  = (1.0 / 3.0) * a2 + (5.0 / 6.0) * a3 + (-1.0 / 6.0) * a4;
+    const double qR2 = (11.0 / 6.0) * a3 + (-7.0 / 6.0) * a4 + (1.0 / 3.0) * a5;
+    const Ind B1 = indicator(d2(a1, a2, a3), a1 - a3);
+    const Ind A2 = indicator(d2(a2, a3, a4), dA(a2, a3, a4));
+    const Ind C3 = indicator(d2(a3, a4, a5), dC(a3, a4, a5));
+    Ind A0, C2;
+    if (WALK) {
+        A0 = w.A0; C2 = w.C2;
+        w.A0 = w.A1; w.A1 = A2; w.C2 = C3;
+    } else {
+        A0 = indicator(d2(a0, a1, a2), dA(a0, a1, a2));
+        C2 = indicator(d2(a2, a3, a4), dC(a2, a3, a4));
+    }
+    vl = wenoz_mix(A0, B1, C2, 1.0 / 10.0, 6.0 / 10.0, 3.0 / 10.0, qL0, qC, qR);
+    vr = wenoz_mix(B1, A2, C3, 3.0 / 10.0, 6.0 / 10.0, 1.0 / 10.0, qC, qR, qR2);
+}
+
+// Whether the face values rule out the shared reciprocals (see above), and
+// whether some velocity needs a full division; both for the whole wave.
+// v_frexp_exp is e for 2^(e-1) <= |x| < 2^e and 0 for zero and NaN.
+__device__ __forceinline__ bool out_of_range(const double (&L)[4], const double (&R)[4], double PL,
+                                             double PR, bool& tiny) {
+    auto e = [](double x) { return __builtin_amdgcn_frexp_exp(x); };
+    const int m = min(min(min(e(L[1]), e(L[2])), e(L[3])), min(min(e(R[1]), e(R[2])), e(R[3])));
+    tiny = __ballot(m < -899) != 0;
+    return __ballot(min(e(PL), e(PR)) < -599 || (m < -199 && (PL == 0.0 || PR == 0.0))) != 0;
+}
+
+// One side of the interface as hllc_normal sees it after its guards
+// (src/hllc.jl:24-59): the energy rebuild of src/euler3d.jl:100-106 uses the
+// same density, |m|^2 (the same sum for x and y sweeps) and kinetic energy.
+template <int DIR>
+struct Side {
+    double r, mn, mt1, mt2, E, KE, vn, p, cs;
+    Recip ir;
+    bool tiny;
+    __device__ __forceinline__ double velocity(double m) const { return tiny ? m / r : quot(m, ir); }
+    __device__ __forceinline__ Side(const double (&W)[4], double P, double g, double gm1, const Recip& ig,
+                                    bool tiny_) : tiny(tiny_) {
+        mn = W[1 + DIR];
+        mt1 = DIR == 0 ? W[2] : W[1];
+        mt2 = DIR == 2 ? W[2] : W[3];
+        // max(rho, 1e-30), also where rho <= 0 resets the side to 1e-30
+        r = W[0] < 1e-30 ? 1e-30 : W[0];
+        ir = recip(r);
+        const double cap = (0.5 * r) * 1e4;
+        double m2 = W[1] * W[1] + W[2] * W[2] + W[3] * W[3];
+        KE = quot(0.5 * m2, ir);
+        KE = cap < KE ? cap : KE;
+        E = quot(P, ig) + KE;
+        if (DIR == 2) {
+            m2 = mn * mn + mt1 * mt1 + mt2 * mt2;
+            KE = quot(0.5 * m2, ir);
+            KE = cap < KE ? cap : KE;
+            E = E < KE ? KE : E;
+        }
+        // rare: a reset or speed-capped side
+        if (__ballot(W[0] <= 0.0 || m2 > (r * r) * 1e4)) {
+            if (W[0] <= 0.0) {
+                mn = 0.0; mt1 = 0.0; mt2 = 0.0; E = 0.0; KE = 0.0;
+            } else if (m2 > (r * r) * 1e4) {
+                const double s = (r * 100.0) / sqrt(m2);
+                mn *= s; mt1 *= s; mt2 *= s;
+                KE = jl_min((0.5 * (mn * mn + mt1 * mt1 + mt2 * mt2)) / r, cap);
+                E = jl_max(E, KE);
+            }
+        }
+        vn = velocity(mn);
+        p = gm1 * (E - KE);
+        cs = sqrt(quot(g * p, ir));
+    }
+};
+
+// src/hllc.jl:60-165 from the guarded sides.
+template <int DIR>
+__device__ __forceinline__ void hllc_shared(const double (&WL)[4], const double (&WR)[4], double PL,
+                                            double PR, double g, double gfac, bool tiny, double F[5]) {
+    const double gm1 = g - 1.0;
+    const Recip ig = recip(gm1);
+    const Side<DIR> l(WL, PL, g, gm1, ig, tiny), r(WR, PR, g, gm1, ig, tiny);
+    double SL, SR;
+    if (l.p > 0.0 && r.p > 0.0) {
+        const double r_avg = 0.5 * (l.r + r.r);
+        const double cs_avg = 0.5 * (l.cs + r.cs);
+        const double x = 0.5 * (l.p + r.p) - ((0.5 * (r.vn - l.vn)) * r_avg) * cs_avg;
+        const double p_star = !(x <= 0.0) ? x : 0.0;
+        const double qL = p_star > l.p ? sqrt(1.0 + gfac * (p_star / l.p - 1.0)) : 1.0;
+        const double qR = p_star > r.p ? sqrt(1.0 + gfac * (p_star / r.p - 1.0)) : 1.0;
+        SL = l.vn - l.cs * qL;
+        SR = r.vn + r.cs * qR;
+    } else {
+        SL = jl_min(l.vn - l.cs, r.vn - r.cs);
+        SR = jl_max(l.vn + l.cs, r.vn + r.cs);
+    }
+    double G[5];
+    const double dL = l.r * (SL - l.vn), dR = r.r * (SR - r.vn);
+    const double denom = dL - dR;
+    const double FmnL = l.r * (l.vn * l.vn) + l.p, FEL = (l.E + l.p) * l.vn;
+    const double FmnR = r.r * (r.vn * r.vn) + r.p, FER = (r.E + r.p) * r.vn;
+    if (fabs(denom) < 1e-100) {
+        G[0] = G[1] = G[2] = G[3] = G[4] = 0.0;
+    } else if (SL >= 0.0) {
+        G[0] = l.mn; G[1] = FmnL; G[2] = l.mt1 * l.vn; G[3] = l.mt2 * l.vn; G[4] = FEL;
+    } else if (SR <= 0.0) {
+        G[0] = r.mn; G[1] = FmnR; G[2] = r.mt1 * r.vn; G[3] = r.mt2 * r.vn; G[4] = FER;
+    } else if ((l.r < r.r ? r.r : l.r) > 3.0 * (r.r < l.r ? r.r : l.r)) {
+        const double inv_dS = 1.0 / (SR - SL);
+        const double SLSR = SL * SR;
+        G[0] = (SR * l.mn - SL * r.mn + SLSR * (r.r - l.r)) * inv_dS;
+        G[1] = (SR * FmnL - SL * FmnR + SLSR * (r.mn - l.mn)) * inv_dS;
+        G[2] = (SR * (l.mt1 * l.vn) - SL * (r.mt1 * r.vn) + SLSR * (r.mt1 - l.mt1)) * inv_dS;
+        G[3] = (SR * (l.mt2 * l.vn) - SL * (r.mt2 * r.vn) + SLSR * (r.mt2 - l.mt2)) * inv_dS;
+        G[4] = (SR * FEL - SL * FER + SLSR * (r.E - l.E)) * inv_dS;
+    } else {
+        const double S_star = ((r.p - l.p) + (l.r * l.vn) * (SL - l.vn) - (r.r * r.vn) * (SR - r.vn)) / denom;
+        auto star = [&](const Side<DIR>& s, double S, double d, double Fmn, double FE) {
+            const double chi = d / (S - S_star);
+            const double Es = fabs(d) > 1e-100
+                                  ? chi * (quot(s.E, s.ir) + (S_star - s.vn) * (S_star + s.p / d)) : 0.0;
+            G[0] = s.mn + S * (chi - s.r);
+            G[1] = Fmn + S * (chi * S_star - s.mn);
+            G[2] = s.mt1 * s.vn + S * (chi * s.velocity(s.mt1) - s.mt1);
+            G[3] = s.mt2 * s.vn + S * (chi * s.velocity(s.mt2) - s.mt2);
+            G[4] = FE + S * (Es - s.E);
+        };
+        if (S_star >= 0.0) star(l, SL, dL, FmnL, FEL);
+        else               star(r, SR, dR, FmnR, FER);
+    }
+    F[0] = G[0];
+    F[1 + DIR] = G[1];
+    F[DIR == 0 ? 2 : 1] = G[2];
+    F[DIR == 2 ? 2 : 3] = G[3];
+    F[4] = G[4];
+}
+
+// The flux of one interface from c and p, or false (for the whole wave) where
+// some lane's values are out of range and the callers take
+// interface_flux_plain.  big: uniform over the wave, a cell of the stencils
+// fails cell_big or gamma gamma_ok.  WALK: w holds the carried indicators and
+// moves on; it is undefined after a refusal.
+template <int DIR, bool WALK>
+__device__ __forceinline__ bool interface_flux_shared(const double (&c)[4][6], const double (&p)[6],
+                                                      double g, double gfac, bool big, double F[5],
+                                                      WenoCarry (&w)[5]) {
+    if (__builtin_expect(big, 0)) return false;
+    double L[4], R[4];
+    // one quantity at a time, as in the split form: the five
+    // reconstructions interleaved need more registers
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        weno5_pair_shared<WALK>(c[q][0], c[q][1], c[q][2], c[q][3], c[q][4], c[q][5], w[q], L[q], R[q]);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    double PLw, PRw;
+    weno5_pair_shared<WALK>(p[0], p[1], p[2], p[3], p[4], p[5], w[4], PLw, PRw);
+    // pressures are +0 or more; where one is NaN so is the reconstruction
+    // that reads it, and the bound does not matter
+    const double mid = hmax(hmax(p[1], p[2]), hmax(p[3], p[4]));
+    const double PL = jl_clamp(PLw, 0.0, hmax(p[0], mid));
+    const double PR = jl_clamp(PRw, 0.0, hmax(mid, p[5]));
+    bool tiny;
+    if (__builtin_expect(out_of_range(L, R, PL, PR, tiny), 0)) return false;
+    __builtin_amdgcn_sched_barrier(0);
+    hllc_shared<DIR>(L, R, PL, PR, g, gfac, tiny, F);
+    return true;
+}
+
+// The carry of the interface whose stencil's first five cells are
+// c[q][M..M+4].
+template <int M = 0>
+__device__ __forceinline__ void interface_walk_start(const double (&c)[4][6], const double (&p)[6],
+                                                     WenoCarry (&w)[5]) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+        weno5_walk_start(c[q][M], c[q][M + 1], c[q][M + 2], c[q][M + 3], c[q][M + 4], w[q]);
+    weno5_walk_start(p[M], p[M + 1], p[M + 2], p[M + 3], p[M + 4], w[4]);
 }
 
 }  // namespace ex
