@@ -168,12 +168,9 @@ static void col_tiles(int nx, int ncross, F&& emit) {
         for (int b = 0; b < ncross; b += 8) emit((64 * (nx / 64)) | COL_HALF, b);
 }
 
-// slots: workgroups the sweep kernel keeps resident (the persistent grid);
-// the y and z walks split each column into runs of one balanced length so
-// that the tile count is a whole multiple of the slots.
 // Reorders a tile list of uneven tiles so that the persistent launch's
-// uniform chunks (workgroup b of G takes tiles [b n / G, (b + 1) n / G), see
-// chunk()) carry about equal work.  A batch of uneven grids gives runs of
+// chunks (n / G tiles per workgroup, the first n % G one more, see chunk())
+// carry about equal work.  A batch of uneven grids gives runs of
 // different lengths, and each grid's tiles sit together, so equal tile
 // counts left some workgroups with several times the work of others.  Tiles
 // go, longest first, to the least loaded chunk that still has room (chunk
@@ -195,7 +192,7 @@ static void balance_chunks(std::vector<Tile>& t, int slots, Weight weight) {
     if (wmax <= 1.1 * wmin) return;
     std::vector<int> cap(G);
     for (int b = 0; b < G; ++b)
-        cap[b] = (int)(((int64_t)(b + 1) * n) / G) - (int)(((int64_t)b * n) / G);
+        cap[b] = n / G + (b < n % G ? 1 : 0);
     std::vector<int> order(n);
     std::iota(order.begin(), order.end(), 0);
     std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return w[a] > w[b]; });
@@ -220,7 +217,57 @@ static void balance_chunks(std::vector<Tile>& t, int slots, Weight weight) {
     t.swap(out);
 }
 
-static std::vector<Tile> flux_tiles(const std::vector<GridDev>& G, int dir, int shape, int slots) {
+// The runs that each grid's columns are cut into (walks and the fused kernel).
+// cols[g] column tiles of len[g] interfaces or cells; a run of L costs L + c (c:
+// its start) and takes at most lmax.  A workgroup's waves share their CU's
+// SIMDs with those of the other resident workgroups, so what matters is the
+// largest sum of runs on a CU; a CU that holds fewer workgroups than fit (occ)
+// finishes them at part of its rate (a lone FP64 walk at 0.87 of two, a lone
+// split walk at about half of four).
+//
+// One grid: the count s of runs per column that minimises that sum over
+// cols * s equal runs, down to runs of 1 where the grid is too small to fill
+// the chip.  (Runs of at least 8 left a 128 x 8 x 8 grid walking its 9 y
+// interfaces in one thread: 46 us against 9.7; rounding s to the nearest count
+// gave a 192^3 grid 576 runs, 2.25 per CU, with the double chunks on one XCD:
+// its FP64 step took 5.41 ms against 4.00.)
+// Several grids: one length for all, from a few candidates, by the mean load
+// of a CU plus half a run for the uneven end.
+static std::vector<int> run_counts(const std::vector<int>& cols, const std::vector<int>& len, double c,
+                                   double lmax, int cus, int occ) {
+    const size_t N = cols.size();
+    std::vector<int> s(N, 1);
+    auto least = [&](int n) { return std::max(1, (int)std::ceil(n / std::min(lmax, (double)ZT_MAX_LEN))); };
+    auto rate = [&](int w) { return std::min(1.0, 0.4 + 0.6 * w / occ); };
+    if (N == 1) {
+        double best = 1e300;
+        for (int k = least(len[0]); k <= len[0]; ++k) {
+            const double run = (len[0] + k - 1) / k + c;
+            const int64_t m = ((int64_t)cols[0] * k + cus - 1) / cus;       // runs on a CU
+            const int rem = (int)(m % occ);
+            const double t = run * ((double)(m - rem) + (rem ? rem / rate(rem) : 0.0));
+            if (t < best) { best = t; s[0] = k; }
+            if (m > 64 * occ) break;                                        // only starts are left to pay
+        }
+        return s;
+    }
+    double best = 1e300;
+    for (double L = std::min(lmax, 96.0); ; L /= 1.25) {
+        std::vector<int> t(N);
+        double work = 0, longest = 0;
+        for (size_t g = 0; g < N; ++g) {
+            t[g] = std::min(len[g], std::max(least(len[g]), (int)(len[g] / L + 0.5)));
+            work += (double)cols[g] * (len[g] + t[g] * c);
+            longest = std::max(longest, (len[g] + t[g] - 1) / t[g] + c);
+        }
+        const double T = std::max(work / cus, longest / rate(1)) + 0.5 * longest;
+        if (T < best) { best = T; s = t; }
+        if (L < 1.0) break;
+    }
+    return s;
+}
+
+static std::vector<Tile> flux_tiles(const std::vector<GridDev>& G, int dir, int shape, int slots, int cus) {
     int W, H;
     flux_shape_dims(dir, shape, W, H);
     std::vector<Tile> t;
@@ -242,36 +289,20 @@ static std::vector<Tile> flux_tiles(const std::vector<GridDev>& G, int dir, int 
         return t;
     }
     if (dir != 0 && flux_walk_len(dir, shape) > 0) {
-        // register walks: column tiles (col_tiles), each column split into
-        // runs along dir.
-        // The persistent launch hands every workgroup the same number of
-        // tiles, so a tile count just above a multiple of the slots leaves
-        // most workgroups idle for a final pass (2304 runs of 32 over 1024
-        // slots take three passes).  The runs of all grids therefore share
-        // one length Lt <= 1.1 * Lmax, chosen so that the column-interfaces
-        // divide evenly over m * slots runs.
-        const int Lmax = flux_walk_len(dir, shape);
-        double work = 0;    // column-interfaces
-        for (const GridDev& d : G)
-            work += (double)col_tile_count(d.nx, dir == 1 ? d.nz : d.ny) *
-                    ((dir == 1 ? d.ny : d.nz) + 1);
-        const double sl = slots > 0 ? slots : 1;
-        int m = (int)std::ceil(work / (sl * Lmax * 1.1));
-        if (m < 1) m = 1;
-        // a batch too small to fill the slots keeps runs of at least 8:
-        // shorter runs would only add window starts
-        const double Lt = std::max(work / (m * sl), 8.0);
+        // register walks: column tiles (col_tiles), each column cut into runs
+        // along dir
+        std::vector<int> cols, len;
+        for (const GridDev& d : G) {
+            cols.push_back(col_tile_count(d.nx, dir == 1 ? d.nz : d.ny));
+            len.push_back((dir == 1 ? d.ny : d.nz) + 1);
+        }
+        const auto runs = run_counts(cols, len, 1.0, 1.1 * flux_walk_len(dir, shape), cus, slots / cus);
         for (int g = 0; g < (int)G.size(); ++g) {
             const GridDev& d = G[g];
-            const int nf = (dir == 1 ? d.ny : d.nz) + 1;      // interfaces along dir
-            const int ncross = dir == 1 ? d.nz : d.ny;
-            int nr = (int)(nf / Lt + 0.5);
-            if (nr < 1) nr = 1;
-            while ((nf + nr - 1) / nr > ZT_MAX_LEN) ++nr;
+            const int nf = len[g], nr = runs[g];
             for (int r = 0; r < nr; ++r) {
                 const int f0 = (int)((int64_t)nf * r / nr), f1 = (int)((int64_t)nf * (r + 1) / nr);
-                if (f1 <= f0) continue;
-                col_tiles(d.nx, ncross, [&](int a, int b) {
+                col_tiles(d.nx, dir == 1 ? d.nz : d.ny, [&](int a, int b) {
                     t.push_back({g, a, b, f0 | ((f1 - f0) << ZT_LEN_SHIFT)});
                 });
             }
@@ -313,34 +344,26 @@ static std::vector<Tile> update_tiles(const std::vector<GridDev>& G) {
 }
 
 // Column tiles of the fused z-sweep + update kernel: 64 x 4 columns of one
-// grid and a run of cells along z.  seg 0/1: runs of 16/32 cells.  seg 2: the
-// runs of each grid have one length (split as evenly as the grid's nz allows),
-// chosen so that the tile count is close to a whole multiple of the slots
-// (resident workgroups) and no run exceeds 96 cells: the persistent launch
-// then gives every workgroup the same work, and long runs amortise the
-// five-cell window start-up.
-static std::vector<Tile> zupdate_tiles(const std::vector<GridDev>& G, int seg, int slots) {
+// grid and a run of cells along z.  seg 0/1: runs of at most 16/32 cells.  seg
+// 2: balanced runs of at most 96 (run_counts; a run of L cells computes L + 1
+// interfaces).
+static std::vector<Tile> zupdate_tiles(const std::vector<GridDev>& G, int seg, int slots, int cus) {
     std::vector<Tile> t;
+    std::vector<int> cols, len;
+    for (const GridDev& d : G) {
+        cols.push_back(col_tile_count(d.nx, d.ny));
+        len.push_back(d.nz);
+    }
     std::vector<int> nseg(G.size(), 1);
     if (seg == 2) {
-        double work = 0;    // column-cells
-        for (const GridDev& d : G) work += (double)col_tile_count(d.nx, d.ny) * d.nz;
-        const double s = slots > 0 ? slots : 1;
-        int m = 1;
-        while (work / (m * s) > 96.0) ++m;
-        const double Lt = work / (m * s);
-        for (size_t g = 0; g < G.size(); ++g) {
-            int n = (int)(G[g].nz / Lt + 0.5);
-            nseg[g] = n < 1 ? 1 : n;
-        }
+        nseg = run_counts(cols, len, 2.0, 96.0, cus, slots / cus);
     } else {
         const int kz = seg == 1 ? 32 : 16;
         for (size_t g = 0; g < G.size(); ++g) nseg[g] = (G[g].nz + kz - 1) / kz;
     }
     for (int g = 0; g < (int)G.size(); ++g) {
         const GridDev& d = G[g];
-        int n = nseg[g];
-        while ((d.nz + n - 1) / n > ZT_MAX_LEN) ++n;
+        const int n = nseg[g];
         for (int s = 0; s < n; ++s) {
             const int k0 = (int)((int64_t)d.nz * s / n), k1 = (int)((int64_t)d.nz * (s + 1) / n);
             if (k1 <= k0) continue;
@@ -375,7 +398,7 @@ static void graph_drop(hipGraphExec_t& e, hipGraph_t& g) {
 
 static int plan_set_shape(Plan& P, int dir, int shape) {
     auto G = host_descs(P);
-    auto t = flux_tiles(G, dir, shape, flux_slots(dir, P.prec, shape, P.ctx->cus));
+    auto t = flux_tiles(G, dir, shape, flux_slots(dir, P.prec, shape, P.ctx->cus), P.ctx->cus);
     CHK(upload_vec(&P.d_ft[dir], t));
     P.nft[dir] = (int)t.size();
     P.shape[dir] = shape;
@@ -433,7 +456,7 @@ static int plan_refresh(Plan& P) {
 
 static int plan_set_zshape(Plan& P, int shape) {
     auto G = host_descs(P);
-    auto t = zupdate_tiles(G, zupdate_seg(shape), zupdate_slots(P.prec, shape, P.ctx->cus));
+    auto t = zupdate_tiles(G, zupdate_seg(shape), zupdate_slots(P.prec, shape, P.ctx->cus), P.ctx->cus);
     CHK(upload_vec(&P.d_zt, t));
     P.nzt = (int)t.size();
     P.zshape = shape;

@@ -72,9 +72,15 @@ __device__ __forceinline__ T bld(const T* base, uint32_t off) {
         return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, NT ? 2 : 0));
 }
 
+// The contiguous tiles of this workgroup.  Where the list does not divide
+// evenly the first workgroups take one more: consecutive workgroups go to
+// different XCDs and CUs, so the longer chunks spread over the chip.  (Chunks
+// cut at b n / G put every longer chunk of, say, 576 tiles over 512 workgroups
+// on the one XCD that workgroups 7, 15, 23, ... run on.)
 __device__ __forceinline__ void chunk(int ntiles, int& t0, int& t1) {
-    t0 = (int)(((int64_t)blockIdx.x * ntiles) / gridDim.x);
-    t1 = (int)(((int64_t)(blockIdx.x + 1) * ntiles) / gridDim.x);
+    const int b = (int)blockIdx.x, q = ntiles / (int)gridDim.x, r = ntiles % (int)gridDim.x;
+    t0 = b * q + min(b, r);
+    t1 = t0 + q + (b < r ? 1 : 0);
 }
 
 // Lane -> (x, row) of a column tile: 64 lanes along x and one row per wave,
@@ -728,32 +734,38 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 4 : 2) void k_fwalk(const Gri
         // applied when the cell is placed, so that the next cell's load stays
         // in flight during the current interface's flux.  A ghost index along
         // the walk reads the active cell it maps to, as load_cell does.
-        auto fetch = [&](int pf) {
-            npf = pf;
+        auto load = [&](int pf, double (&u)[5]) {
             int sp_ = pf;
             if (G.lmode & 1) sp_ = bc_src(pf, DIR == 1 ? G.ny : G.nz, G.bc & (DIR == 1 ? 2 : 4));
             const int64_t base = DIR == 1 ? ((int64_t)(NG + cc0) * G.Ny + sp_) * G.pitch + BSN_XOFF
                                           : ((int64_t)sp_ * G.Ny + NG + cc0) * G.pitch + BSN_XOFF;
 #pragma unroll
-            for (int q = 0; q < 5; ++q) nxt[q] = bld<double, true>(G.U + q * G.fs + base, uoff);
+            for (int q = 0; q < 5; ++q) u[q] = bld<double, true>(G.U + q * G.fs + base, uoff);
         };
-        auto place = [&](int slot) {
-            if ((G.lmode & 2) && npf >= NG && npf < NG + (DIR == 1 ? G.ny : G.nz))
-                apply_floor<FAST>(nxt, G.rho_floor, G.P_floor, G.gamma);
-            const double pr = Prec<T>::pressure(nxt, G.gamma);
-            big |= __ballot(Prec<T>::big_cell(nxt, pr)) != 0;
+        auto fetch = [&](int pf) { npf = pf; load(pf, nxt); };
+        auto place = [&](int slot, int pf, double (&u)[5]) {
+            if ((G.lmode & 2) && pf >= NG && pf < NG + (DIR == 1 ? G.ny : G.nz))
+                apply_floor<FAST>(u, G.rho_floor, G.P_floor, G.gamma);
+            const double pr = Prec<T>::pressure(u, G.gamma);
+            big |= __ballot(Prec<T>::big_cell(u, pr)) != 0;
 #pragma unroll
-            for (int q = 0; q < 4; ++q) c[q][slot] = (T)nxt[q];
+            for (int q = 0; q < 4; ++q) c[q][slot] = (T)u[q];
             p[slot] = (T)pr;
         };
+        {
+            // the window's cells in one memory round trip
+            double u[5][5];
 #pragma unroll
-        for (int m = 0; m < 5; ++m) { fetch(f0 + m); place(m); }
-        fetch(f0 + 5);
+            for (int m = 0; m < 5; ++m) load(f0 + m, u[m]);
+            fetch(f0 + 5);
+#pragma unroll
+            for (int m = 0; m < 5; ++m) place(m, f0 + m, u[m]);
+        }
         typename Prec<T>::Carry wc[5];
         Prec<T>::start(c, p, wc);
         const int fend = f0 + len;
         auto step = [&](int f) {
-            place(5);                                   // cell f+5 (padded)
+            place(5, npf, nxt);                         // cell f+5 (padded)
             if (f + 1 < fend) fetch(f + 6);             // in flight during the flux
             T F[5];
             Prec<T>::template flux<DIR, true>(c, p, G, big, F, wc);
@@ -1086,30 +1098,30 @@ __global__ __launch_bounds__(256, WB) void k_zupdate(const GridDev* __restrict__
             // streaming loads (2.7 % on this kernel at 256^3 against cached
             // loads; the x and y fluxes, whose faces neighbouring lanes and
             // rows share, stay cached)
-            auto fetch = [&](int pz) {
-                npz = pz;
+            auto load = [&](int pz, double (&v)[5]) {
                 // load_cell along z: a ghost plane reads the active plane its
                 // index maps to; without the ring an active cell is floored here
                 const int sk = (G.lmode & 1) ? bc_src(pz, G.nz, G.bc & 4) : pz;
                 const double* const b = G.U + sk * zs;
 #pragma unroll
-                for (int q = 0; q < 5; ++q) nxt[q] = bld<double, true>(b + q * G.fs, uo);
+                for (int q = 0; q < 5; ++q) v[q] = bld<double, true>(b + q * G.fs, uo);
                 if (!RING && (G.lmode & 2) && pz >= NG && pz < NG + G.nz)
-                    apply_floor<FAST>(nxt, G.rho_floor, G.P_floor, G.gamma);
+                    apply_floor<FAST>(v, G.rho_floor, G.P_floor, G.gamma);
             };
-            auto place = [&](int slot) {
+            auto fetch = [&](int pz) { npz = pz; load(pz, nxt); };
+            auto place = [&](int slot, int pz, double (&v)[5]) {
                 if (RING) {
-                    // raw value (unfloored) into the ring; slot npz & 3 is not
-                    // read again before cell npz + 4 replaces it
+                    // raw value (unfloored) into the ring; slot pz & 3 is not
+                    // read again before cell pz + 4 replaces it
 #pragma unroll
-                    for (int q = 0; q < 5; ++q) ring[npz & 3][q][rt] = nxt[q];
-                    if ((G.lmode & 2) && npz >= NG && npz < NG + G.nz)
-                        apply_floor<FAST>(nxt, G.rho_floor, G.P_floor, G.gamma);
+                    for (int q = 0; q < 5; ++q) ring[pz & 3][q][rt] = v[q];
+                    if ((G.lmode & 2) && pz >= NG && pz < NG + G.nz)
+                        apply_floor<FAST>(v, G.rho_floor, G.P_floor, G.gamma);
                 }
-                const double pr = Prec<T>::pressure(nxt, G.gamma);
-                big |= __ballot(Prec<T>::big_cell(nxt, pr)) != 0;
+                const double pr = Prec<T>::pressure(v, G.gamma);
+                big |= __ballot(Prec<T>::big_cell(v, pr)) != 0;
 #pragma unroll
-                for (int q = 0; q < 4; ++q) c[q][slot] = (T)nxt[q];
+                for (int q = 0; q < 4; ++q) c[q][slot] = (T)v[q];
                 p[slot] = (T)pr;
             };
             T fx[2][5], fy[2][5];
@@ -1142,16 +1154,22 @@ __global__ __launch_bounds__(256, WB) void k_zupdate(const GridDev* __restrict__
                     cell_state<FAST>(G, cc, stage, u, un);
                 }
             };
+            {
+                // the window's cells in one memory round trip
+                double v[5][5];
 #pragma unroll
-            for (int m = 0; m < 5; ++m) { fetch(k0 + m); place(m); }
-            fetch(k0 + 5);
+                for (int m = 0; m < 5; ++m) load(k0 + m, v[m]);
+                fetch(k0 + 5);
+#pragma unroll
+                for (int m = 0; m < 5; ++m) place(m, k0 + m, v[m]);
+            }
             // split form: the smoothness indicators that consecutive
             // interfaces share are carried along the column
             typename Prec<T>::Carry wc[5];
             if constexpr (CARRY) Prec<T>::start(c, p, wc);
             T fz0[5];                                   // the previous interface's z flux
             for (int f = k0; f <= kend; ++f) {
-                place(5);                               // cell f+5
+                place(5, npz, nxt);                     // cell f+5
                 if (PF >= 1 && f < kend) fetch(f + 6);  // next iteration's cell, in flight during the flux
                 const int k = f - 1;                    // the cell finished in this iteration
                 if (PF == 1 && f > k0) operands(k);
