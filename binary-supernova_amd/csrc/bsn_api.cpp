@@ -151,21 +151,47 @@ struct bsn_fmr {
 // Tile lists
 
 // Column tiles of a grid's (x, cross) plane for the y/z walks and the fused
-// kernel: workgroups of 64 x 4 (x, rows) and, where a grid's rows end 32
-// cells or fewer into their last x-tile, half-width workgroups of 32 x 8 for
-// that tile (COL_HALF), so that the lanes past the row end do not idle.
-static int col_tile_count(int nx, int ncross) {
-    const int rem = nx % 64, nfull = nx / 64 + (rem > 32 ? 1 : 0);
-    return nfull * ((ncross + 3) / 4) + (rem > 0 && rem <= 32 ? (ncross + 7) / 8 : 0);
+// kernel, cross = z for the y walk (dir 1) and y otherwise: workgroups of 64 x 4
+// (x, rows), whose rows start on cache lines, or flat ones of 256 consecutive
+// columns (COL_FLAT) where rows that do not fill their last 64 lanes, or a
+// row count that does not fill its last workgroup, would idle more than
+// FLAT_GAIN of the lanes.  Flat rows of the split form, whose kernels wait on
+// memory, are padded to 16 columns so that every 16 lanes read whole lines: on
+// 48 grids of random sizes from 32 to 128 the step took 7.32 ms, 7.98 unpadded
+// and 7.58 with 64 x 4 tiles alone.  FP64 rows are not padded: 12 such grids
+// 2.19 ms against 2.31 with 64 x 4 tiles.  Between 5 and 10 % of idle lanes
+// (nx = 116 to 120) both take the same time.
+static const double FLAT_GAIN = 0.07;
+static int col_cross(const GridDev& d, int dir) { return dir == 1 ? d.nz : d.ny; }
+static int64_t col_width(const GridDev& d) { return col_width(d.nx, d.prec); }
+
+static bool col_flat(const GridDev& d, int dir) {
+    const int64_t ncross = col_cross(d, dir);
+    const int64_t blocked = 256 * ((d.nx + 63) / 64) * ((ncross + 3) / 4);
+    const int64_t flat = 256 * ((col_width(d) * ncross + 255) / 256);
+    if ((double)flat > (1.0 - FLAT_GAIN) * (double)blocked) return false;
+    // the y walk's lanes address the z planes their wave wraps into through
+    // 32-bit offsets from its first
+    const int64_t planes = 63 / col_width(d) + 2;
+    return dir != 1 || planes * ((int64_t)d.Ny + 1) * std::max(d.pitch, d.fp[1]) * 8 < ((int64_t)1 << 31);
+}
+
+static int col_tile_count(const GridDev& d, int dir) {
+    const int64_t ncross = col_cross(d, dir);
+    return col_flat(d, dir) ? (int)((col_width(d) * ncross + 255) / 256)
+                            : (d.nx + 63) / 64 * (int)((ncross + 3) / 4);
 }
 
 template <typename F>
-static void col_tiles(int nx, int ncross, F&& emit) {
-    const int rem = nx % 64, nfull = nx / 64 + (rem > 32 ? 1 : 0);
+static void col_tiles(const GridDev& d, int dir, F&& emit) {
+    const int ncross = col_cross(d, dir);
+    if (col_flat(d, dir)) {
+        const int64_t w = col_width(d), n = w * ncross;
+        for (int64_t e = 0; e < n; e += 256) emit((int)(e % w) | COL_FLAT, (int)(e / w));
+        return;
+    }
     for (int b = 0; b < ncross; b += 4)
-        for (int t = 0; t < nfull; ++t) emit(64 * t, b);
-    if (rem > 0 && rem <= 32)
-        for (int b = 0; b < ncross; b += 8) emit((64 * (nx / 64)) | COL_HALF, b);
+        for (int a = 0; a < d.nx; a += 64) emit(a, b);
 }
 
 // Reorders a tile list of uneven tiles so that the persistent launch's
@@ -221,9 +247,10 @@ static void balance_chunks(std::vector<Tile>& t, int slots, Weight weight) {
 // cols[g] column tiles of len[g] interfaces or cells; a run of L costs L + c (c:
 // its start) and takes at most lmax.  A workgroup's waves share their CU's
 // SIMDs with those of the other resident workgroups, so what matters is the
-// largest sum of runs on a CU; a CU that holds fewer workgroups than fit (occ)
-// finishes them at part of its rate (a lone FP64 walk at 0.87 of two, a lone
-// split walk at about half of four).
+// largest sum of runs on a CU; a CU that holds w workgroups where occ fit works
+// at lone + (1 - lone) w / occ of its rate.  The split kernels wait on memory
+// and need their waves more: lone 0.2 gave 64^3 0.378 ms for two steps, 0.4
+// 0.401; FP64 0.4 0.601 ms, 0.75 0.622.
 //
 // One grid: the count s of runs per column that minimises that sum over
 // cols * s equal runs, down to runs of 1 where the grid is too small to fill
@@ -234,11 +261,12 @@ static void balance_chunks(std::vector<Tile>& t, int slots, Weight weight) {
 // Several grids: one length for all, from a few candidates, by the mean load
 // of a CU plus half a run for the uneven end.
 static std::vector<int> run_counts(const std::vector<int>& cols, const std::vector<int>& len, double c,
-                                   double lmax, int cus, int occ) {
+                                   double lmax, int cus, int occ, int prec) {
     const size_t N = cols.size();
     std::vector<int> s(N, 1);
     auto least = [&](int n) { return std::max(1, (int)std::ceil(n / std::min(lmax, (double)ZT_MAX_LEN))); };
-    auto rate = [&](int w) { return std::min(1.0, 0.4 + 0.6 * w / occ); };
+    const double lone = prec == BSN_PREC_FP64 ? 0.4 : 0.2;
+    auto rate = [&](int w) { return std::min(1.0, lone + (1.0 - lone) * w / occ); };
     if (N == 1) {
         double best = 1e300;
         for (int k = least(len[0]); k <= len[0]; ++k) {
@@ -293,16 +321,17 @@ static std::vector<Tile> flux_tiles(const std::vector<GridDev>& G, int dir, int 
         // along dir
         std::vector<int> cols, len;
         for (const GridDev& d : G) {
-            cols.push_back(col_tile_count(d.nx, dir == 1 ? d.nz : d.ny));
+            cols.push_back(col_tile_count(d, dir));
             len.push_back((dir == 1 ? d.ny : d.nz) + 1);
         }
-        const auto runs = run_counts(cols, len, 1.0, 1.1 * flux_walk_len(dir, shape), cus, slots / cus);
+        const auto runs = run_counts(cols, len, 1.0, 1.1 * flux_walk_len(dir, shape), cus, slots / cus,
+                                     G[0].prec);
         for (int g = 0; g < (int)G.size(); ++g) {
             const GridDev& d = G[g];
             const int nf = len[g], nr = runs[g];
             for (int r = 0; r < nr; ++r) {
                 const int f0 = (int)((int64_t)nf * r / nr), f1 = (int)((int64_t)nf * (r + 1) / nr);
-                col_tiles(d.nx, dir == 1 ? d.nz : d.ny, [&](int a, int b) {
+                col_tiles(d, dir, [&](int a, int b) {
                     t.push_back({g, a, b, f0 | ((f1 - f0) << ZT_LEN_SHIFT)});
                 });
             }
@@ -351,12 +380,12 @@ static std::vector<Tile> zupdate_tiles(const std::vector<GridDev>& G, int seg, i
     std::vector<Tile> t;
     std::vector<int> cols, len;
     for (const GridDev& d : G) {
-        cols.push_back(col_tile_count(d.nx, d.ny));
+        cols.push_back(col_tile_count(d, 2));
         len.push_back(d.nz);
     }
     std::vector<int> nseg(G.size(), 1);
     if (seg == 2) {
-        nseg = run_counts(cols, len, 2.0, 96.0, cus, slots / cus);
+        nseg = run_counts(cols, len, 2.0, 96.0, cus, slots / cus, G[0].prec);
     } else {
         const int kz = seg == 1 ? 32 : 16;
         for (size_t g = 0; g < G.size(); ++g) nseg[g] = (G[g].nz + kz - 1) / kz;
@@ -368,7 +397,7 @@ static std::vector<Tile> zupdate_tiles(const std::vector<GridDev>& G, int seg, i
             const int k0 = (int)((int64_t)d.nz * s / n), k1 = (int)((int64_t)d.nz * (s + 1) / n);
             if (k1 <= k0) continue;
             const int c = k0 | ((k1 - k0) << ZT_LEN_SHIFT);
-            col_tiles(d.nx, d.ny, [&](int a, int b) { t.push_back({g, a, b, c}); });
+            col_tiles(d, 2, [&](int a, int b) { t.push_back({g, a, b, c}); });
         }
     }
     // a run of L cells reads a window of L + 5

@@ -82,10 +82,14 @@ struct Tile {
     int g, a, b, c;
 };
 
-// Column tiles (the y/z walks and the fused z-sweep + update) flag in a a
-// half-width tile: 32 lanes along x and 8 rows per workgroup instead of 64 and
-// 4, for the last x-tile of a grid whose rows end 32 cells or fewer into it.
-#define COL_HALF (1 << 30)
+// Column tiles (the y/z walks and the fused z-sweep + update) flag in a a flat
+// tile: 256 consecutive columns in row-major order instead of 64 x 4, over rows
+// of col_width columns.
+#define COL_FLAT (1 << 30)
+#ifdef __HIPCC__
+__host__ __device__
+#endif
+static inline int col_width(int nx, int prec) { return prec ? (nx + 15) & ~15 : nx; }
 
 // Fused z-sweep + update tiles pack the first cell and the column length in c.
 #define ZT_K0_MASK 0x1FFFFF

@@ -84,12 +84,20 @@ __device__ __forceinline__ void chunk(int ntiles, int& t0, int& t1) {
 }
 
 // Lane -> (x, row) of a column tile: 64 lanes along x and one row per wave,
-// or, for a half-width tile (COL_HALF in a), 32 lanes along x and two rows per
-// wave.  Uniform over the workgroup.
-__device__ __forceinline__ void col_lane(int a, int b, int& i, int& row) {
-    const int lx = threadIdx.x & 63, ly = threadIdx.x >> 6;
-    if (a & COL_HALF) { i = (a & ~COL_HALF) + (lx & 31); row = b + 2 * ly + (lx >> 5); }
-    else              { i = a + lx; row = b + ly; }
+// or, in a flat tile (COL_FLAT in a), 256 consecutive columns in row-major
+// order from (a, b), wrapping after width columns.  row0: the wave's first row.
+__device__ __forceinline__ void col_lane(int width, int a, int b, int& i, int& row, int& row0) {
+    const int lx = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (a & COL_FLAT) {
+        const unsigned s = (unsigned)(a & ~COL_FLAT) + 64u * wv, q0 = s / (unsigned)width;
+        const unsigned x = s - q0 * width + lx, q = x / (unsigned)width;
+        row0 = b + (int)q0;
+        row = row0 + (int)q;
+        i = (int)(x - q * width);
+    } else {
+        row0 = row = b + wv;
+        i = a + lx;
+    }
 }
 
 __device__ __forceinline__ int find_grid(const int64_t* __restrict__ off, int ngrids, int64_t e) {
@@ -712,13 +720,11 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 4 : 2) void k_fwalk(const Gri
         const Tile tl = tiles[t];
         const GridDev& G = grids[tl.g];
         const int f0 = tl.c & ZT_K0_MASK, len = tl.c >> ZT_LEN_SHIFT;
-        int i, cc;
-        col_lane(tl.a, tl.b, i, cc);
-        // the wave's first row (uniform) and this lane's row past it (0, or 1
-        // in the second half of a half-width tile): the walk's addresses are
-        // a scalar base per cell or face and a lane offset fixed for the tile
-        const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-        const int cc0 = (tl.a & COL_HALF) ? tl.b + 2 * wv : tl.b + wv;
+        // the wave's first row cc0 (uniform) and this lane's row past it: the
+        // walk's addresses are a scalar base per cell or face and a lane offset
+        // fixed for the tile
+        int i, cc, cc0;
+        col_lane(col_width(G.nx, FAST), tl.a, tl.b, i, cc, cc0);
         const int dr = cc - cc0;
         if (i >= G.nx || cc >= (DIR == 1 ? G.nz : G.ny)) continue;
         const uint32_t uoff =
@@ -1076,8 +1082,8 @@ __global__ __launch_bounds__(256, WB) void k_zupdate(const GridDev* __restrict__
         const GridDev& G = grids[tl.g];
         // tile.c packs the first cell k0 (bits 0-20) and the column length (bits 21-30)
         const int k0 = tl.c & ZT_K0_MASK, klen = tl.c >> ZT_LEN_SHIFT;
-        int i, j;
-        col_lane(tl.a, tl.b, i, j);
+        int i, j, j0;
+        col_lane(col_width(G.nx, FAST), tl.a, tl.b, i, j, j0);
         uint64_t smax = 0;
         if (i < G.nx && j < G.ny) {
             const int kend = min(k0 + klen, G.nz);
