@@ -101,6 +101,7 @@ struct Plan {
     int prec = 0;
     GridDev* d_grids = nullptr;
     int shape[3] = {0, 0, 0};
+    int kshape[3] = {0, 0, 0};   // as launch_flux takes it (FLUX_XFLAT)
     Tile* d_ft[3] = {nullptr, nullptr, nullptr};
     int nft[3] = {0, 0, 0};
     Tile* d_ut = nullptr;
@@ -174,6 +175,17 @@ static bool col_flat(const GridDev& d, int dir) {
     // 32-bit offsets from its first
     const int64_t planes = 63 / col_width(d) + 2;
     return dir != 1 || planes * ((int64_t)d.Ny + 1) * std::max(d.pitch, d.fp[1]) * 8 < ((int64_t)1 << 31);
+}
+
+// The same choice for the x sweep's 64 x 4 tiles, whose edge tiles take the last
+// interface of 256 rows.  48 split grids of random sizes from 32 to 128 took
+// 6.98 ms per step with flat x tiles, 7.32 without; 96 x 128 x 128 0.504 ms
+// against 0.534.
+static bool x_flat(const GridDev& d) {
+    if (d.nx < 8 || d.ny < XFLAT_ROWS) return false;
+    const int64_t blocked = d.nz * (256LL * ((d.nx + 63) / 64) * ((d.ny + 3) / 4) + 256 * ((d.ny + 255) / 256));
+    const int64_t flat = 256 * (((int64_t)(d.nx + 1) * d.ny * d.nz + 255) / 256);
+    return (double)flat <= (1.0 - FLAT_GAIN) * (double)blocked;
 }
 
 static int col_tile_count(const GridDev& d, int dir) {
@@ -342,7 +354,13 @@ static std::vector<Tile> flux_tiles(const std::vector<GridDev>& G, int dir, int 
     }
     for (int g = 0; g < (int)G.size(); ++g) {
         const GridDev& d = G[g];
-        if (dir == 0) {
+        if (dir == 0 && W == 64 && x_flat(d)) {
+            const int64_t n = (int64_t)(d.nx + 1) * d.ny * d.nz;
+            for (int64_t e = 0; e < n; e += 256) {
+                const int64_t row = e / (d.nx + 1);
+                t.push_back({g, (int)(e % (d.nx + 1)) | COL_FLAT, (int)(row % d.ny), (int)(row / d.ny)});
+            }
+        } else if (dir == 0) {
             for (int k = 0; k < d.nz; ++k) {
                 for (int j0 = 0; j0 < d.ny; j0 += H)
                     for (int f0 = 0; f0 < d.nx; f0 += W) t.push_back({g, f0, j0, k});
@@ -430,7 +448,10 @@ static int plan_set_shape(Plan& P, int dir, int shape) {
     auto t = flux_tiles(G, dir, shape, flux_slots(dir, P.prec, shape, P.ctx->cus), P.ctx->cus);
     CHK(upload_vec(&P.d_ft[dir], t));
     P.nft[dir] = (int)t.size();
-    P.shape[dir] = shape;
+    P.shape[dir] = P.kshape[dir] = shape;
+    if (dir == 0 && shape == 0)
+        for (const GridDev& d : G)
+            if (x_flat(d)) P.kshape[0] = FLUX_XFLAT;
     graph_drop(P.gexec, P.graph);
     return BSN_OK;
 }
@@ -540,13 +561,14 @@ static int plan_new(bsn_ctx* ctx, const std::vector<bsn_grid*>& grids, Plan** ou
         if (g->h.prec != P->prec) { delete P; return set_err(BSN_ERR_ARG, "grids of mixed precision"); }
         if (g->ctx != ctx) { delete P; return set_err(BSN_ERR_ARG, "grids of different contexts"); }
     }
-    // starting shapes (kept until bsn_batch_autotune or set_*shape*): y and z
-    // register walks in balanced runs (the autotuner's choice from 32^3
-    // batches to the 256^3 box), the fused kernel with the LDS ring, the
-    // early load and balanced runs; the x sweep tiled (64x4 split, 16x16
-    // FP64), which unlike the x walks keeps its lanes busy on narrow grids.
-    if (P->prec == 1) { P->shape[0] = 0; P->shape[1] = FLUX_WALK_SHAPE0 + 2; P->shape[2] = FLUX_WALK_SHAPE0 + 2; P->zshape = 11; }
-    else              { P->shape[0] = 2; P->shape[1] = FLUX_WALK_SHAPE0 + 2; P->shape[2] = FLUX_WALK_SHAPE0 + 2; P->zshape = 11; }
+    // starting shapes (kept until bsn_batch_autotune or set_*shape*): the x
+    // sweep in 64 x 4 or flat tiles, y and z register walks in balanced runs,
+    // the fused kernel with the LDS ring, the early load and balanced runs (the
+    // autotuner's choice from 32^3 batches to the 256^3 box).  FP64 grids of 192^3
+    // took 3.95 ms per step with 64 x 4 x tiles, 4.12 with 16 x 16.
+    P->shape[0] = 0;
+    P->shape[1] = P->shape[2] = FLUX_WALK_SHAPE0 + 2;
+    P->zshape = 11;
     int r = plan_build(*P);
     if (r != BSN_OK) { plan_free(P); return r; }
     *out = P;
@@ -570,7 +592,7 @@ static int plan_fluxes(Plan& P, const GridDev* table = nullptr, int ndirs = 3) {
     if (!table) table = P.d_grids;
     for (int d = 0; d < ndirs; ++d) {
         prof_mark(P, d);
-        HIPCHK(launch_flux(L, d, P.prec, P.shape[d], table, P.d_ft[d], P.nft[d], 0));
+        HIPCHK(launch_flux(L, d, P.prec, P.kshape[d], table, P.d_ft[d], P.nft[d], 0));
     }
     prof_mark(P, 9);
     return BSN_OK;
@@ -1636,7 +1658,7 @@ static int plan_autotune(Plan& P, std::string& out) {
         const GridDev* T = P.d_st[stage - 1];
         for (int k : {0, 1, 3}) {
             if (e && k == which) HIPCHK(hipEventRecord(e[0], L.stream));
-            if (k < 3) HIPCHK(launch_flux(L, k, P.prec, P.shape[k], T, P.d_ft[k], P.nft[k], 0));
+            if (k < 3) HIPCHK(launch_flux(L, k, P.prec, P.kshape[k], T, P.d_ft[k], P.nft[k], 0));
             else       HIPCHK(launch_zupdate(L, P.prec, P.zshape, T, P.d_zt, P.nzt, stage, 0));
             if (e && k == which) HIPCHK(hipEventRecord(e[1], L.stream));
         }

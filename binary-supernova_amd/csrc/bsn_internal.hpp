@@ -91,6 +91,12 @@ __host__ __device__
 #endif
 static inline int col_width(int nx, int prec) { return prec ? (nx + 15) & ~15 : nx; }
 
+// Flat x tiles (COL_FLAT in a): 256 consecutive x interfaces, nx + 1 per row,
+// rows in (j, k) order, from interface a of row (b, c).  A wave's 64 touch at
+// most XFLAT_ROWS rows, which the x extent (at least 8) ensures; the y extent is
+// at least XFLAT_ROWS.
+#define XFLAT_ROWS 8
+
 // Fused z-sweep + update tiles pack the first cell and the column length in c.
 #define ZT_K0_MASK 0x1FFFFF
 #define ZT_LEN_SHIFT 21

@@ -374,7 +374,7 @@ __device__ __forceinline__ void store_face(const GridDev& G, const T (&F)[5], in
     for (int q = 0; q < 5; ++q) __builtin_nontemporal_store(F[q], &Fp[q * G.ffs[DIR] + o]);
 }
 
-template <int DIR, typename T, int W, int H>
+template <int DIR, typename T, int W, int H, bool FLAT = false>
 __global__ __launch_bounds__(W * H, (DIR == 0 && W == 64 && H == 4 && sizeof(T) == 4) ? 6 : 1) void k_flux(const GridDev* __restrict__ grids,
                                                  const Tile* __restrict__ tiles, int ntiles) {
     constexpr int NT = W * H;
@@ -386,7 +386,12 @@ __global__ __launch_bounds__(W * H, (DIR == 0 && W == 64 && H == 4 && sizeof(T) 
     // held to 80 VGPRs, 6 waves per SIMD (a few values spilled): 0.367 ms
     // against 0.376 at 91 VGPRs, 5 waves.
     constexpr bool WAVE = DIR == 0 && W * H == 256 && (W == 64 || W == 32 || W == 16);
-    __shared__ T lds[5][SA][SB];
+    // FLAT (64 x 4): the list may hold flat tiles.  A kernel of its own, used
+    // where a grid of the list has them: 64 x 4 tiles took 0.379 ms in it at
+    // 256^3 (split) against 0.363.
+    static_assert(!FLAT || (DIR == 0 && W == 64 && H == 4), "flat tiles are 4 waves of 64");
+    constexpr int LW = 64 + 5 * XFLAT_ROWS;      // staged cells of a wave, FLAT
+    __shared__ T lds[5][FLAT ? H : SA][FLAT ? LW : SB];
     const int tid = threadIdx.x;
     int t0, t1;
     chunk(ntiles, t0, t1);
@@ -422,7 +427,113 @@ __global__ __launch_bounds__(W * H, (DIR == 0 && W == 64 && H == 4 && sizeof(T) 
             }
             continue;
         }
-        if constexpr (WAVE) {
+        if constexpr (FLAT) {
+            // each wave stages and computes 64 consecutive interfaces: of one
+            // row, or, in a flat tile, of up to XFLAT_ROWS rows in row-major
+            // order, each row's n interfaces with the n + 5 cells they read.
+            // Cell t of the wave's sequence goes to slot t; the interface of a
+            // lane in the wave's row s reads slots lane + 5 s ...  Both loads
+            // of a lane are issued before either is used (indices clamped into
+            // the grid), then floors and pressures.  The wave's first row is
+            // uniform: its base stays in scalar registers.
+            const int wv = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+            const bool flat = tl.a & COL_FLAT;
+            int x0 = tl.a & ~COL_FLAT, j0 = tl.b, k0 = tl.c;
+            // per staged cell: its padded x, byte offset from the first row's
+            // start and whether it exists; of the lane's interface: f and s
+            int pc[2], f, seg = 0;
+            uint32_t ro[2] = {0, 0};
+            bool ok[2], mine;
+            const double* rowU;
+            if (flat) {
+                for (x0 += 64 * wv; x0 > G.nx; x0 -= G.nx + 1)
+                    if (++j0 == G.ny) { j0 = 0; ++k0; }
+                const int n0 = G.nx + 1 - x0;            // interfaces left in the first row
+                // t / d as a product: exact for t < 128 and d >= 9
+                const uint32_t m6 = 65536u / (uint32_t)(G.nx + 6) + 1, m1 = 65536u / (uint32_t)(G.nx + 1) + 1;
+                auto past = [&](int l) { return l < n0 ? 0 : 1 + (int)(((uint32_t)(l - n0) * m1) >> 16); };
+                // a row past the first wraps into the next plane at most once
+                // (flat tiles come from grids of at least XFLAT_ROWS rows)
+                auto row_ok = [&](int s) { return (j0 + s < G.ny ? k0 : k0 + 1) < G.nz; };
+                const int tmax = 64 + 5 * (past(63) + 1);
+                seg = past(lane);
+                f = seg ? lane - n0 - (seg - 1) * (G.nx + 1) : x0 + lane;
+                mine = row_ok(seg);
+#pragma unroll
+                for (int r = 0; r < 2; ++r) {
+                    const int t = lane + 64 * r, v = t - (n0 + 5);
+                    const int sg = v < 0 ? 0 : 1 + (int)(((uint32_t)v * m6) >> 16);
+                    pc[r] = v < 0 ? x0 + t : v - (sg - 1) * (G.nx + 6);
+                    ok[r] = t < tmax && row_ok(sg);
+                    // rows of one plane are a pitch apart, the next plane
+                    // starts 2 NG rows on
+                    ro[r] = ok[r] ? (uint32_t)(sg + (j0 + sg >= G.ny ? 2 * NG : 0)) * (uint32_t)G.pitch * 8u : 0u;
+                    pc[r] = ok[r] ? pc[r] : 0;
+                }
+                rowU = G.U + uidx(G, 0, j0 + NG, min(k0, G.nz - 1) + NG);
+            } else {
+                // a row's last interface belongs to the edge tiles
+                j0 += wv;
+                f = x0 + lane;
+                const bool row = j0 < G.ny;
+                mine = row && f < G.nx;
+#pragma unroll
+                for (int r = 0; r < 2; ++r) {
+                    pc[r] = min(x0 + (r ? W + min(lane, 4) : lane), Nx - 1);
+                    ok[r] = row && (r == 0 || lane < 5) && x0 + W * r + lane < Nx;
+                }
+                rowU = G.U + uidx(G, 0, min(j0, G.ny - 1) + NG, k0 + NG);
+            }
+            double u[2][5];
+            bool big = Prec<T>::big_gamma(G.gamma);
+#pragma unroll
+            for (int r = 0; r < 2; ++r) {
+                const int pi = (G.lmode & 1) ? bc_src(pc[r], G.nx, G.bc & 1) : pc[r];
+#pragma unroll
+                for (int q = 0; q < 5; ++q) u[r][q] = bld(rowU + q * G.fs, ro[r] + (uint32_t)pi * 8u);
+            }
+#pragma unroll
+            for (int r = 0; r < 2; ++r) {
+                if (ok[r]) {
+                    if ((G.lmode & 2) && pc[r] >= NG && pc[r] < NG + G.nx)
+                        apply_floor<FAST>(u[r], G.rho_floor, G.P_floor, G.gamma);
+                    const double pr = Prec<T>::pressure(u[r], G.gamma);
+                    big |= Prec<T>::big_cell(u[r], pr);
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) lds[q][wv][lane + 64 * r] = (T)u[r][q];
+                    lds[4][wv][lane + 64 * r] = (T)pr;
+                }
+            }
+            // the cells come from other lanes of this wave: the LDS runs one
+            // wave's operations in order, and the fences keep the compiler
+            // from moving the reads above the writes
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            const bool wbig = __ballot(big) != 0;        // any cell of the wave
+            if (mine) {
+                const int l0 = lane + 5 * seg;
+#pragma unroll
+                for (int m = 0; m < 6; ++m) {
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) c[q][m] = lds[q][wv][l0 + m];
+                    p[m] = lds[4][wv][l0 + m];
+                }
+                T F[5];
+                Prec<T>::template flux_at<0>(c, p, G, wbig, F, nc,
+                                             [&](int q, int m) { return lds[q][wv][l0 + m]; });
+                T* rowF = (T*)G.F[0] + ((int64_t)k0 * G.ny + j0) * G.fp[0];
+                const uint32_t fo = (uint32_t)(seg * G.fp[0] + f) * (uint32_t)sizeof(T);
+#pragma unroll
+                for (int q = 0; q < 5; ++q)
+                    __builtin_nontemporal_store(F[q], at_off(rowF + q * G.ffs[0], fo));
+            }
+            // the next tile's stores follow this tile's reads (same order)
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            continue;
+        } else if constexpr (WAVE) {
             // each wave stages and computes its own RW = 64 / W rows of the
             // tile (lane -> row hb + lane / W, x = lane % W): cells f0 .. f0+W+4
             // of each row, both loads issued before either is used (indices
@@ -1832,14 +1943,14 @@ static int occupancy_grid(const void* fn, int threads, size_t lds, int ntiles, i
     return (int)(g < 1 ? 1 : g);
 }
 
-template <int DIR, typename T, int W, int H>
+template <int DIR, typename T, int W, int H, bool FLAT = false>
 static hipError_t launch_flux_t(const LaunchCtx& L, const GridDev* grids, const Tile* tiles,
                                 int ntiles, int max_wg) {
     if (ntiles <= 0) return hipSuccess;
-    const void* fn = (const void*)&k_flux<DIR, T, W, H>;
+    const void* fn = (const void*)&k_flux<DIR, T, W, H, FLAT>;
     int g = occupancy_grid(fn, W * H, 0, ntiles, L.cus);
     if (max_wg > 0 && g > max_wg) g = max_wg;
-    hipLaunchKernelGGL((k_flux<DIR, T, W, H>), dim3(g), dim3(W * H), 0, L.stream, grids, tiles, ntiles);
+    hipLaunchKernelGGL((k_flux<DIR, T, W, H, FLAT>), dim3(g), dim3(W * H), 0, L.stream, grids, tiles, ntiles);
     return hipGetLastError();
 }
 
@@ -1870,7 +1981,7 @@ static hipError_t launch_flux_shape(const LaunchCtx& L, int shape, const GridDev
                                     const Tile* tiles, int ntiles, int max_wg) {
     if (DIR != 0 && shape >= FLUX_WALK_SHAPE0)
         return launch_fwalk_t<DIR == 0 ? 1 : DIR, T>(L, grids, tiles, ntiles, max_wg);
-    if (DIR == 0 && shape >= FLUX_XWALK_SHAPE0)
+    if (DIR == 0 && shape >= FLUX_XWALK_SHAPE0 && shape != FLUX_XFLAT)
         switch (shape - FLUX_XWALK_SHAPE0) {
             case 0: return launch_fxwalk_t<T, 2, true>(L, grids, tiles, ntiles, max_wg);
             case 1: return launch_fxwalk_t<T, 4, true>(L, grids, tiles, ntiles, max_wg);
@@ -1880,6 +1991,7 @@ static hipError_t launch_flux_shape(const LaunchCtx& L, int shape, const GridDev
     // 4: 32x16
     if (DIR == 0) {
         switch (shape) {
+            case FLUX_XFLAT: return launch_flux_t<0, T, 64, 4, true>(L, grids, tiles, ntiles, max_wg);
             case 1: return launch_flux_t<DIR, T, 32, 8>(L, grids, tiles, ntiles, max_wg);
             case 2: return launch_flux_t<DIR, T, 16, 16>(L, grids, tiles, ntiles, max_wg);
             default: return launch_flux_t<DIR, T, 64, 4>(L, grids, tiles, ntiles, max_wg);

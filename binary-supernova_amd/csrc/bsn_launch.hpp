@@ -18,6 +18,8 @@ struct LaunchCtx {
 // of 16, 32 or 64 interfaces.
 #define FLUX_XWALK_SHAPE0 3
 #define FLUX_WALK_SHAPE0 5
+// launch_flux only: x shape 0 (64 x 4) on a list that holds flat tiles
+#define FLUX_XFLAT 256
 void flux_shape_dims(int dir, int shape, int& W, int& H);
 int flux_shape_count(int dir);
 int flux_walk_len(int dir, int shape);

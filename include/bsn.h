@@ -235,8 +235,7 @@ int bsn_batch_destroy(bsn_batch* b);
 /* Times every tile shape of every kernel on the current states and keeps the
  * fastest; writes a JSON report of the choice into report (may be NULL).
  * Without it a batch (and every FMR level and single-grid call) starts from
- * the shapes the autotuner keeps for a 256^3 box: split x 0, y/z 2, fused
- * kernel 11; FP64 x 2, y/z 2, fused kernel 2. */
+ * x 0, y/z 7 and fused kernel 11. */
 int bsn_batch_autotune(bsn_batch* b, char* report, int report_len);
 /* Sets the flux shape ids explicitly (x: 0..2 tiled, 3..5 walks of 2, 4 and 4
  * interfaces per lane through LDS-staged rows, the last storing its fluxes
