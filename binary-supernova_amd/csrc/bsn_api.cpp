@@ -2044,18 +2044,13 @@ static int fmr_refresh(bsn_fmr* m) {
     return BSN_OK;
 }
 
-static int64_t ghost_total(const GridDev& d) {
-    return 2 * BSN_NG * ((int64_t)d.Ny * d.Nz + (int64_t)d.nx * d.Nz + (int64_t)d.nx * d.ny);
-}
-
 // interp: from the parent state interpolated in time (fmr_interp), else from
 // the parent's current state.
 static int fmr_prolong(bsn_fmr* m, int l, int all_cells, bool interp,
                        ProlongDst dst = ProlongDst{0, {}}) {
     const GridDev& C = m->lev[l]->h;
     const GridDev& Pg = m->lev[l - 1]->h;
-    const int64_t total = all_cells ? (int64_t)(C.nx + 2 * BSN_NG) * C.Ny * C.Nz : ghost_total(C);
-    HIPCHK(launch_prolong(m->ctx->L(), m->d_all, m->d_f + (l - 1), total,
+    HIPCHK(launch_prolong(m->ctx->L(), m->d_all, m->d_f + (l - 1), C, m->hf[l - 1].ratio,
                           interp ? m->hf[l - 1].Uci : Pg.U, interp ? m->hf[l - 1].Ucit : nullptr,
                           all_cells, dst));
     return BSN_OK;

@@ -97,6 +97,42 @@ static inline int col_width(int nx, int prec) { return prec ? (nx + 15) & ~15 : 
 // at least XFLAT_ROWS.
 #define XFLAT_ROWS 8
 
+// Work of a prolongation (k_prolong): the child's x, y and z ghost slabs (or, all
+// cells, one list in place of the z slabs) in groups of at most 2 x 2 fine cells
+// with one coarse centre in the slab's plane; n? groups, in blocks of 64 of
+// their own.
+#ifdef __HIPCC__
+#define BSN_HD __host__ __device__
+#else
+#define BSN_HD
+#endif
+struct ProlongWork {
+    int gx, gy, gyg, gzg;     // groups along x and y, and along y and z with their ghosts
+    int64_t nx, ny, nz, bx, by, bz;
+};
+
+// along an axis of n cells, with its ghosts or without
+BSN_HD static inline int fine_groups(int n, int ghosts, int r) {
+    const int g = ghosts ? BSN_NG : 0;
+    return ((n + g - 1) / r + (g + r - 1) / r + 1) * ((r + 1) / 2);
+}
+
+BSN_HD static inline ProlongWork prolong_work(int nx, int ny, int nz, int all_cells, int r) {
+    ProlongWork w;
+    w.gx = fine_groups(nx, all_cells, r);
+    w.gy = fine_groups(ny, all_cells, r);
+    w.gyg = fine_groups(ny, 1, r);
+    w.gzg = fine_groups(nz, 1, r);
+    const int64_t layers = 2 * BSN_NG;
+    w.nx = all_cells ? 0 : layers * w.gyg * w.gzg;
+    w.ny = all_cells ? 0 : layers * w.gx * w.gzg;
+    w.nz = (all_cells ? nz + layers : layers) * w.gx * w.gy;
+    w.bx = (w.nx + 63) / 64;
+    w.by = (w.ny + 63) / 64;
+    w.bz = (w.nz + 63) / 64;
+    return w;
+}
+
 // Fused z-sweep + update tiles pack the first cell and the column length in c.
 #define ZT_K0_MASK 0x1FFFFF
 #define ZT_LEN_SHIFT 21

@@ -22,6 +22,7 @@
 // chunk of the list, which keeps neighbouring tiles (shared halo cells) on one
 // CU and one XCD L2.
 #include <hip/hip_runtime.h>
+#include <algorithm>
 #include <mutex>
 #include "bsn_internal.hpp"
 #include "bsn_physics.hpp"
@@ -114,10 +115,6 @@ __device__ __forceinline__ int find_grid(const int64_t* __restrict__ off, int ng
 // slabs: x-slabs (ghost i, all j, k), y-slabs (active i, ghost j, all k) and
 // z-slabs (active i, j, ghost k) -- the same partition as the reference's
 // fill order (euler3d.jl:36-43, fmr3d.jl:228-254).
-
-__device__ __forceinline__ int64_t ghost_count(const GridDev& G) {
-    return 2 * NG * ((int64_t)G.Ny * G.Nz + (int64_t)G.nx * G.Nz + (int64_t)G.nx * G.ny);
-}
 
 __device__ __forceinline__ void ghost_decode(const GridDev& G, int64_t t, int& i, int& j, int& k) {
     const int64_t A = 2 * NG * (int64_t)G.Ny * G.Nz;
@@ -1576,115 +1573,186 @@ __global__ void k_totals_final(const double* __restrict__ part, int nblocks, dou
 }
 
 // ---------------------------------------------------------------------------
-// FMR transfer operators (src/fmr3d.jl).  Coarse index arithmetic follows
-// _coarse_stencil (fmr3d.jl:165-170) in FP64 with ties-to-even rounding.
+// FMR transfer operators (src/fmr3d.jl).  Fine active cell a (0-based) of a box
+// that starts at coarse cell lo has the stencil centre lo + floor(a / ratio) and
+// the weights of a mod ratio: what _coarse_stencil (fmr3d.jl:165-170) computes
+// in FP64, where no centre is nearer than 1 / (2 ratio) to a tie.
 
-__device__ __forceinline__ void coarse_stencil(int ig_f1, int c_lo, int ratio, int& ic0, int& sx) {
-    // ig_f1 is the reference's 1-based fine index
-    const double xi = ((double)c_lo - 0.5) + ((double)(ig_f1 - NG) - 0.5) / (double)ratio;
-    const double r = rint(xi);
-    ic0 = (int)r;
-    int s = (int)floor(((xi - r) + 0.5) * (double)ratio);
-    sx = s < 0 ? 0 : (s > ratio - 1 ? ratio - 1 : s);
+// Fine cells of one axis, 0-based from the first active one, in groups of at most
+// two that share a coarse centre: cells a0 .. a1 - 1, coarse cells from c0.
+struct FineAxis {
+    int a0, a1, c0, p;           // p: groups of a coarse cell
+};
+
+__device__ __forceinline__ FineAxis fine_axis(int n, bool ghosts, int r) {
+    FineAxis x;
+    x.a0 = ghosts ? -NG : 0;
+    x.a1 = n + (ghosts ? NG : 0);
+    x.c0 = x.a0 < 0 ? -((r - 1 - x.a0) / r) : 0;
+    x.p = (r + 1) / 2;
+    return x;
 }
 
-// Prolongation of fine cells from the parent state interpolated in time,
-// Uc(alpha) = (1 - alpha) Ucn + alpha Ucnp1 (fmr3d.jl:551), evaluated per
-// coarse value on the fly.  all_cells = 1 fills every fine cell
-// (_prolong_all!), else only ghost cells in the reference's slab partition.
-// The values go to each of the dst.n buffers in the child's layout, or to
-// the child's state when dst.n is 0.
-__global__ void k_prolong(const GridDev* __restrict__ grids, const FmrDev* __restrict__ fmr,
-                          const double* __restrict__ Uca, const double* __restrict__ Ucat,
-                          int all_cells, ProlongDst dst) {
+// Prolongation of up to NX x NY x NZ fine cells around one coarse centre, whose
+// 125 coarse values src (at the stencil's first cell; sx, sy, sz: strides, fs:
+// field stride) serve them all.  w?: the Lagrange weights of each axis's first
+// cell, those of a second one 5 on.  Each cell and field sums its terms in the
+// reference's (di, dj, dk) order.  The next 25 values are in flight while the
+// last 25 are summed.
+template <int NX, int NY, int NZ, typename Put>
+__device__ __forceinline__ void prolong_cells(const double* __restrict__ src, int64_t sx, int64_t sy,
+                                              int64_t sz, int64_t fs, const double* wx, const double* wy,
+                                              const double* wz, Put&& put) {
+    double val[NX][NY][NZ][5] = {};
+    double nxt[5][5], wi[NX], wj[NY], wk[NZ][5];
+    auto load = [&](int di, int dj) {
+        const double* b = src + di * sx + dj * sy;
+#pragma unroll
+        for (int dk = 0; dk < 5; ++dk)
+#pragma unroll
+            for (int q = 0; q < 5; ++q) nxt[dk][q] = b[dk * sz + q * fs];
+#pragma unroll
+        for (int x = 0; x < NX; ++x) wi[x] = wx[5 * x + di];
+#pragma unroll
+        for (int y = 0; y < NY; ++y) wj[y] = wy[5 * y + dj];
+    };
+#pragma unroll
+    for (int z = 0; z < NZ; ++z)
+#pragma unroll
+        for (int dk = 0; dk < 5; ++dk) wk[z][dk] = wz[5 * z + dk];
+    load(0, 0);
+    int di = 0, dj = 0;
+#pragma unroll 1
+    for (int m = 0; m < 25; ++m) {
+        double cur[5][5], wij[NX][NY];
+#pragma unroll
+        for (int dk = 0; dk < 5; ++dk)
+#pragma unroll
+            for (int q = 0; q < 5; ++q) cur[dk][q] = nxt[dk][q];
+#pragma unroll
+        for (int x = 0; x < NX; ++x)
+#pragma unroll
+            for (int y = 0; y < NY; ++y) wij[x][y] = wi[x] * wj[y];
+        if (++dj == 5) { dj = 0; ++di; }
+        if (m < 24) load(di, dj);
+#pragma unroll
+        for (int dk = 0; dk < 5; ++dk)
+#pragma unroll
+            for (int x = 0; x < NX; ++x)
+#pragma unroll
+                for (int y = 0; y < NY; ++y)
+#pragma unroll
+                    for (int z = 0; z < NZ; ++z) {
+                        const double w = wij[x][y] * wk[z][dk];
+#pragma unroll
+                        for (int q = 0; q < 5; ++q) val[x][y][z][q] += w * cur[dk][q];
+                    }
+    }
+#pragma unroll
+    for (int x = 0; x < NX; ++x)
+#pragma unroll
+        for (int y = 0; y < NY; ++y)
+#pragma unroll
+            for (int z = 0; z < NZ; ++z) put(x, y, z, val[x][y][z]);
+}
+
+// Prolongation of fine cells from the parent state Uca (fmr3d.jl:551: the one
+// interpolated in time).  all_cells = 1 fills every fine cell (_prolong_all!),
+// else only ghost cells in the reference's slab partition.  The values go to
+// each of the dst.n buffers in the child's layout, or to the child's state when
+// dst.n is 0.
+//
+// Bound by the 625 coarse values a cell gathers through L1 and L2: a thread takes
+// the 2 x 2 fine cells in its slab's plane that share a coarse centre, for a
+// quarter of the loads, and no wave takes cells of two slabs (it would run
+// both).  A child of 128 x 128 x 96 took 100 us per call cell for cell, 71 with waves
+// that mix slabs, now 62; with 1 x 2 cells 77 (twice the loads).
+__global__ __launch_bounds__(64) void k_prolong(const GridDev* __restrict__ grids, const FmrDev* __restrict__ fmr,
+                                                const double* __restrict__ Uca, const double* __restrict__ Ucat,
+                                                int all_cells, ProlongDst dst) {
     const FmrDev& M = *fmr;
     const GridDev& C = grids[M.parent];
     const GridDev& Fg = grids[M.child];
-    const int Nfx = Fg.nx + 2 * NG;
-    const int64_t total = all_cells ? (int64_t)Nfx * Fg.Ny * Fg.Nz : ghost_count(Fg);
-    for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < total;
-         e += (int64_t)gridDim.x * blockDim.x) {
-        int i, j, k;
-        // x-slab ghost cells read the transposed copy when there is one: their
-        // lanes then run along y, where consecutive cells are adjacent in it
-        const bool xt = !all_cells && Ucat && e < 2 * NG * (int64_t)Fg.Ny * Fg.Nz;
-        if (all_cells) {
-            i = (int)(e % Nfx);
-            const int64_t r = e / Nfx;
-            j = (int)(r % Fg.Ny); k = (int)(r / Fg.Ny);
-        } else if (xt) {
-            j = (int)(e % Fg.Ny);
-            const int64_t r = e / Fg.Ny;
-            k = (int)(r % Fg.Nz);
-            const int ig = (int)(r / Fg.Nz);
-            i = ig < NG ? ig : Fg.nx + ig;
-        } else {
-            ghost_decode(Fg, e, i, j, k);
-        }
-        int ic0, jc0, kc0, si, sj, sk;
-        coarse_stencil(i + 1, M.lo[0], M.ratio, ic0, si);
-        coarse_stencil(j + 1, M.lo[1], M.ratio, jc0, sj);
-        coarse_stencil(k + 1, M.lo[2], M.ratio, kc0, sk);
-        const int64_t d = uidx(Fg, i, j, k);
-        if (xt) {
-            // the same terms in the same order, from the transposed box
-            const int bx = M.phi[0] - M.plo[0] + 1, by = M.phi[1] - M.plo[1] + 1;
-            const int bz = M.phi[2] - M.plo[2] + 1;
-            const int64_t bt = (int64_t)bx * by * bz;
-            double val[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-            for (int di = -2; di <= 2; ++di) {
-                const int ig = NG + ic0 + di - 1 - M.plo[0];
-                const double wi = M.w[si * 5 + di + 2];
-                for (int dj = -2; dj <= 2; ++dj) {
-                    const int jg = NG + jc0 + dj - 1 - M.plo[1];
-                    const double wij = wi * M.w[sj * 5 + dj + 2];
-                    const int64_t ob = ((int64_t)ig * bz + (NG + kc0 - 3 - M.plo[2])) * by + jg;
-#pragma unroll
-                    for (int dk = 0; dk < 5; ++dk) {
-                        const int64_t o = ob + (int64_t)dk * by;
-                        const double w = wij * M.w[sk * 5 + dk];
-#pragma unroll
-                        for (int q = 0; q < 5; ++q) val[q] += w * Ucat[q * bt + o];
-                    }
-                }
-            }
-            if (dst.n == 0) {
-#pragma unroll
-                for (int q = 0; q < 5; ++q) Fg.U[q * Fg.fs + d] = val[q];
-            }
-            for (int b = 0; b < dst.n; ++b) {
-#pragma unroll
-                for (int q = 0; q < 5; ++q) dst.p[b][q * Fg.fs + d] = val[q];
-            }
-            continue;
-        }
-        const int64_t zs = (int64_t)C.Ny * C.pitch;
-        // the five fields accumulate side by side; each field's terms are
-        // summed in the reference's (di, dj, dk) order
-        double val[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-        for (int di = -2; di <= 2; ++di) {
-            const int ig = NG + ic0 + di - 1;
-            const double wi = M.w[si * 5 + di + 2];
-            for (int dj = -2; dj <= 2; ++dj) {
-                const int jg = NG + jc0 + dj - 1;
-                const double wij = wi * M.w[sj * 5 + dj + 2];
-                const int64_t ob = uidx(C, ig, jg, NG + kc0 - 3);
-#pragma unroll
-                for (int dk = 0; dk < 5; ++dk) {
-                    const int64_t o = ob + dk * zs;
-                    const double w = wij * M.w[sk * 5 + dk];
-#pragma unroll
-                    for (int q = 0; q < 5; ++q) val[q] += w * Uca[q * C.fs + o];
-                }
-            }
-        }
+    const int r = M.ratio;
+    const ProlongWork W = prolong_work(Fg.nx, Fg.ny, Fg.nz, all_cells, r);
+    const FineAxis X = fine_axis(Fg.nx, all_cells, r), Yg = fine_axis(Fg.ny, true, r);
+    const FineAxis Y = fine_axis(Fg.ny, all_cells, r), Zg = fine_axis(Fg.nz, true, r);
+    const int64_t zs = (int64_t)C.Ny * C.pitch;
+    // the coarse cell and the weights of fine cell a (a >= -NG)
+    auto centre = [&](int a, int& c, const double*& w) {
+        c = (a + NG * r) / r - NG;
+        w = M.w + 5 * (a - c * r);
+    };
+    auto group = [&](const FineAxis& x, int g, int& c, int& a, const double*& w) {
+        c = x.c0 + g / x.p;
+        a = c * r + 2 * (g % x.p);
+        w = M.w + 5 * (a - c * r);
+    };
+    auto in = [&](const FineAxis& x, int a, int c) { return a >= x.a0 && a < min(x.a1, (c + 1) * r); };
+    auto ghost = [](int l, int n) { return l < NG ? l - NG : n + l - NG; };
+    auto store = [&](int i, int j, int k, const double (&v)[5]) {
+        const int64_t d = uidx(Fg, NG + i, NG + j, NG + k);
         if (dst.n == 0) {
 #pragma unroll
-            for (int q = 0; q < 5; ++q) Fg.U[q * Fg.fs + d] = val[q];
+            for (int q = 0; q < 5; ++q) Fg.U[q * Fg.fs + d] = v[q];
         }
         for (int b = 0; b < dst.n; ++b) {
 #pragma unroll
-            for (int q = 0; q < 5; ++q) dst.p[b][q * Fg.fs + d] = val[q];
+            for (int q = 0; q < 5; ++q) dst.p[b][q * Fg.fs + d] = v[q];
+        }
+    };
+    // the stencil's first cell (padded, 0-based) in the parent
+    auto first = [&](int a, int c) { return NG + M.lo[a] + c - 3; };
+    for (int64_t blk = blockIdx.x; blk < W.bx + W.by + W.bz; blk += gridDim.x) {
+        int cx, cy, cz, i, j, k;
+        const double *wx, *wy, *wz;
+        if (blk < W.bx) {
+            // x slabs: lanes along y, from the transposed box, when there is
+            // one, where consecutive y cells are adjacent
+            const int64_t e = blk * 64 + threadIdx.x;
+            if (e >= W.nx) continue;
+            const uint32_t u = (uint32_t)e, t = u / (uint32_t)W.gyg;
+            group(Yg, (int)(u % (uint32_t)W.gyg), cy, j, wy);
+            group(Zg, (int)(t % (uint32_t)W.gzg), cz, k, wz);
+            i = ghost((int)(t / (uint32_t)W.gzg), Fg.nx);
+            centre(i, cx, wx);
+            const int pi = first(0, cx), pj = first(1, cy), pk = first(2, cz);
+            const double* src = Uca + uidx(C, pi, pj, pk);
+            int64_t sx = 1, sy = C.pitch, sz = zs, fs = C.fs;
+            if (Ucat) {
+                sy = 1;
+                sz = M.phi[1] - M.plo[1] + 1;
+                sx = sz * (M.phi[2] - M.plo[2] + 1);
+                fs = sx * (M.phi[0] - M.plo[0] + 1);
+                src = Ucat + (pi - M.plo[0]) * sx + (pk - M.plo[2]) * sz + (pj - M.plo[1]);
+            }
+            prolong_cells<1, 2, 2>(src, sx, sy, sz, fs, wx, wy, wz, [&](int, int y, int z, const double (&v)[5]) {
+                if (in(Yg, j + y, cy) && in(Zg, k + z, cz)) store(i, j + y, k + z, v);
+            });
+        } else if (blk < W.bx + W.by) {
+            const int64_t e = (blk - W.bx) * 64 + threadIdx.x;
+            if (e >= W.ny) continue;
+            const uint32_t u = (uint32_t)e, t = u / (uint32_t)W.gx;
+            group(X, (int)(u % (uint32_t)W.gx), cx, i, wx);
+            j = ghost((int)(t % (2 * NG)), Fg.ny);
+            centre(j, cy, wy);
+            group(Zg, (int)(t / (2 * NG)), cz, k, wz);
+            prolong_cells<2, 1, 2>(Uca + uidx(C, first(0, cx), first(1, cy), first(2, cz)), 1, C.pitch, zs, C.fs,
+                                   wx, wy, wz, [&](int x, int, int z, const double (&v)[5]) {
+                if (in(X, i + x, cx) && in(Zg, k + z, cz)) store(i + x, j, k + z, v);
+            });
+        } else {
+            const int64_t e = (blk - W.bx - W.by) * 64 + threadIdx.x;
+            if (e >= W.nz) continue;
+            const uint32_t u = (uint32_t)e, t = u / (uint32_t)W.gx;
+            group(X, (int)(u % (uint32_t)W.gx), cx, i, wx);
+            group(Y, (int)(t % (uint32_t)W.gy), cy, j, wy);
+            k = all_cells ? (int)(t / (uint32_t)W.gy) - NG : ghost((int)(t / (uint32_t)W.gy), Fg.nz);
+            centre(k, cz, wz);
+            prolong_cells<2, 2, 1>(Uca + uidx(C, first(0, cx), first(1, cy), first(2, cz)), 1, C.pitch, zs, C.fs,
+                                   wx, wy, wz, [&](int x, int y, int, const double (&v)[5]) {
+                if (in(X, i + x, cx) && in(Y, j + y, cy)) store(i + x, j + y, k, v);
+            });
         }
     }
 }
@@ -2272,11 +2340,12 @@ hipError_t launch_totals(const LaunchCtx& L, const GridDev& G, double* part, int
     return hipGetLastError();
 }
 
-hipError_t launch_prolong(const LaunchCtx& L, const GridDev* grids, const FmrDev* fmr, int64_t total,
-                          const double* Uca, const double* Ucat, int all_cells, ProlongDst dst) {
-    if (total <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_prolong, dim3(flat_blocks(total, L.cus)), dim3(256), 0, L.stream, grids, fmr,
-                       Uca, Ucat, all_cells, dst);
+hipError_t launch_prolong(const LaunchCtx& L, const GridDev* grids, const FmrDev* fmr, const GridDev& child,
+                          int ratio, const double* Uca, const double* Ucat, int all_cells, ProlongDst dst) {
+    // blocks of one wave: few threads with much work each, spread over all CUs
+    const ProlongWork w = prolong_work(child.nx, child.ny, child.nz, all_cells, ratio);
+    hipLaunchKernelGGL(k_prolong, dim3((unsigned)std::min<int64_t>(w.bx + w.by + w.bz, 64LL * L.cus)), dim3(64), 0, L.stream,
+                       grids, fmr, Uca, Ucat, all_cells, dst);
     return hipGetLastError();
 }
 

@@ -71,8 +71,8 @@ struct ProlongDst {
 };
 // Ucat: the interpolated parent box transposed (FmrDev.Ucit) for the x-slab
 // ghost cells, or null to read Uca for every cell.
-hipError_t launch_prolong(const LaunchCtx& L, const GridDev* grids, const FmrDev* fmr, int64_t total,
-                          const double* Uca, const double* Ucat, int all_cells,
+hipError_t launch_prolong(const LaunchCtx& L, const GridDev* grids, const FmrDev* fmr, const GridDev& child,
+                          int ratio, const double* Uca, const double* Ucat, int all_cells,
                           ProlongDst dst = ProlongDst{0, {}});
 hipError_t launch_time_interp(const LaunchCtx& L, const GridDev* grids, const FmrDev* fmr,
                               int64_t total, double alpha);
