@@ -1972,6 +1972,8 @@ extern "C" int bsn_fmr_create(bsn_ctx* ctx, int nlevels, bsn_grid* const* levels
             const int nca = a == 0 ? ch.nx : a == 1 ? ch.ny : ch.nz;
             f.plo[a] = BSN_NG + coarse_centre(1, f.lo[a], f.ratio) - 3;
             f.phi[a] = BSN_NG + coarse_centre(nca + 2 * BSN_NG, f.lo[a], f.ratio) + 1;
+            f.slo[a] = BSN_NG + coarse_centre(BSN_NG, f.lo[a], f.ratio) + 1;
+            f.shi[a] = BSN_NG + coarse_centre(nca + BSN_NG + 1, f.lo[a], f.ratio) - 3;
         }
         if (hipMalloc((void**)&f.Uci, 5 * levels[l]->h.fs * 8) != hipSuccess)
             return fail(set_err(BSN_ERR_HIP, "interpolation buffer allocation"));
@@ -2004,30 +2006,32 @@ extern "C" int bsn_fmr_destroy(bsn_fmr* m) {
     return BSN_OK;
 }
 
-// Stage tables of the fused level step.  Level buffers: U (the state), Un
-// (its raw copy at the start of the step, the RK3 base state and, for a
-// parent, the start state its child interpolates from), W1 and W2 (work):
+// Stage tables of the fused level step.  Level buffers: U (the state, until
+// stage 3 overwrites it cell by cell also the RK3 base state), W1 and W2 (work):
 // stage 1 reads U and writes W1, stage 2 reads W1 and writes W2, stage 3
-// reads W2 and writes U, so U ends with the new state and Un keeps the old
-// one as in the in-place step.  The root maps ghost cells to active cells
+// reads W2 and writes U.  Un keeps what is read of the old state beyond that
+// (launch_level_begin): the fourth table, for the ghost combination, takes a
+// child's ghost cells from it.  The root maps ghost cells to active cells
 // under its boundary conditions on load; a child reads the ghost cells
-// prolonged into each stage's input buffer.  Stage 1 floors active cells on
+// prolonged into each stage input.  Stage 1 floors active cells on
 // load (the start-of-stage floors).
 static int fmr_stage_tables(bsn_fmr* m) {
-    if (m->d_fst.empty()) m->d_fst.assign(3 * m->nlev, nullptr);
+    if (m->d_fst.empty()) m->d_fst.assign(4 * m->nlev, nullptr);
     for (int l = 0; l < m->nlev; ++l) {
         bsn_grid* g = m->lev[l];
         CHK(ensure_work(g));
         CHK(ensure_work2(g));
         const int map = l == 0 ? 1 : 0;
         GridDev d = g->h;
-        d.Un = g->h.Un;
-        GridDev st[3] = {d, d, d};
+        d.Un = g->h.U;
+        GridDev st[4] = {d, d, d, d};
         st[0].lmode = map | 2; st[0].U = g->h.U;   st[0].Uout = g->d_work;
         st[1].lmode = map;     st[1].U = g->d_work; st[1].Uout = g->d_work2;
         st[2].lmode = map;     st[2].U = g->d_work2; st[2].Uout = g->h.U;
-        for (int s = 0; s < 3; ++s) {
-            GridDev*& t = m->d_fst[3 * l + s];
+        st[3] = st[2];
+        if (l > 0) st[3].Un = g->h.Un;
+        for (int s = 0; s < 4; ++s) {
+            GridDev*& t = m->d_fst[4 * l + s];
             if (!t) HIPCHK(hipMalloc((void**)&t, sizeof(GridDev)));
             HIPCHK(hipMemcpy(t, &st[s], sizeof(GridDev), hipMemcpyHostToDevice));
         }
@@ -2075,12 +2079,13 @@ static int fmr_advance(bsn_fmr* m, int l) {
     const LaunchCtx L = m->ctx->L();
     const bool child = l + 1 < m->nlev;
     const GridDev& h = m->lev[l]->h;
-    if (child) HIPCHK(launch_fr_zero(L, m->d_f + l, m->hf[l].froff[6]));
+    const FmrDev* const df = child ? m->d_f + l : nullptr;
+    const FmrDev* const hf = child ? &m->hf[l] : nullptr;
+    HIPCHK(launch_level_begin(L, m->d_all, l, h, df, hf, l > 0 && !m->inplace));
     if (!m->inplace) {
         // fused form: per stage the x and y sweeps, then the z sweep fused
         // with the update (storing the z faces the registers read), then the
         // flux-register sums of the stage; same bits as the in-place form
-        HIPCHK(launch_copy_state(L, h, h.U, h.Un));
         if (l > 0) {
             // alpha and the interpolated parent are fixed for the sub-cycle,
             // so the ghost cells of all three stage inputs are prolonged once
@@ -2089,7 +2094,7 @@ static int fmr_advance(bsn_fmr* m, int l) {
             CHK(fmr_prolong(m, l, 0, true, ProlongDst{3, {g->h.U, g->d_work, g->d_work2}}));
         }
         for (int s = 1; s <= 3; ++s) {
-            const GridDev* T = m->d_fst[3 * l + s - 1];
+            const GridDev* T = m->d_fst[4 * l + s - 1];
             CHK(plan_fluxes(P, T, 2));
             prof_mark(P, 3);
             HIPCHK(launch_zupdate(L, P.prec, P.zshape, T, P.d_zt, P.nzt, s, 0));
@@ -2097,7 +2102,7 @@ static int fmr_advance(bsn_fmr* m, int l) {
             if (child) HIPCHK(launch_fr_coarse(L, P.prec, m->d_all, m->d_f + l, m->hf[l].froff[6] / 5, RK_W[s - 1]));
             if (l > 0) HIPCHK(launch_fr_fine(L, P.prec, m->d_all, m->d_f + (l - 1), m->hf[l - 1].froff[6] / 5, RK_W[s - 1]));
         }
-        CHK(plan_ghost_combine(P, 3, m->d_fst[3 * l + 2]));
+        CHK(plan_ghost_combine(P, 3, m->d_fst[4 * l + 3]));
     } else {
     if (l > 0) HIPCHK(launch_copy_state(L, h, h.U, h.Un));
     if (l > 0) CHK(fmr_interp(m, l));
@@ -2126,7 +2131,7 @@ static int fmr_advance(bsn_fmr* m, int l) {
         const int64_t ncells = (int64_t)(f.hi[0] - f.lo[0] + 1) * (f.hi[1] - f.lo[1] + 1) * (f.hi[2] - f.lo[2] + 1);
         HIPCHK(launch_restrict(L, m->d_all, m->d_f + l, ncells));
         HIPCHK(launch_bc_correct(L, m->d_all, m->d_f + l, f.froff[6] / 5));
-        CHK(plan_floors(P, 0));
+        HIPCHK(launch_floors_box(L, m->d_all, m->d_f + l, f));
     }
     return BSN_OK;
 }

@@ -152,4 +152,6 @@ struct FmrDev {
     double* Uci;              // parent state interpolated in time (parent layout)
     double* Ucit;             // the same over the plo..phi box, y fastest, then z, then x
     int plo[3], phi[3];       // padded parent cells any prolongation stencil reads
+    int slo[3], shi[3];       // the ghost slabs' stencils read those at most slo or at
+                              // least shi along the slab's axis (the box's shell)
 };

@@ -116,6 +116,10 @@ __device__ __forceinline__ int find_grid(const int64_t* __restrict__ off, int ng
 // z-slabs (active i, j, ghost k) -- the same partition as the reference's
 // fill order (euler3d.jl:36-43, fmr3d.jl:228-254).
 
+__device__ __forceinline__ int64_t ghost_count(const GridDev& G) {
+    return 2 * NG * ((int64_t)G.Ny * G.Nz + (int64_t)G.nx * G.Nz + (int64_t)G.nx * G.ny);
+}
+
 __device__ __forceinline__ void ghost_decode(const GridDev& G, int64_t t, int& i, int& j, int& k) {
     const int64_t A = 2 * NG * (int64_t)G.Ny * G.Nz;
     const int64_t B = 2 * NG * (int64_t)G.nx * G.Nz;
@@ -247,6 +251,23 @@ __device__ __forceinline__ void load_cell(const GridDev& G, int i, int j, int k,
     if (FLOOR && (G.lmode & 2) && active) apply_floor<FAST>(u, G.rho_floor, G.P_floor, G.gamma);
 }
 
+__device__ __forceinline__ void floor_cell(const GridDev& G, int64_t c, bool copy_un) {
+    double u[5];
+#pragma unroll
+    for (int q = 0; q < 5; ++q) u[q] = G.U[q * G.fs + c];
+    if (copy_un) {
+#pragma unroll
+        for (int q = 0; q < 5; ++q) G.Un[q * G.fs + c] = u[q];
+    }
+    // the split form floors with the same division wherever it floors
+    const bool fired = G.prec == 1 ? apply_floor<true>(u, G.rho_floor, G.P_floor, G.gamma)
+                                   : apply_floor<false>(u, G.rho_floor, G.P_floor, G.gamma);
+    if (fired) {
+#pragma unroll
+        for (int q = 0; q < 5; ++q) G.U[q * G.fs + c] = u[q];
+    }
+}
+
 // Floors on active cells (apply_floors_3d!, euler3d.jl:73-80); with copy_un
 // the raw value is saved to Un first.
 __global__ void k_floors(const GridDev* __restrict__ grids, const int64_t* __restrict__ off,
@@ -260,21 +281,7 @@ __global__ void k_floors(const GridDev* __restrict__ grids, const int64_t* __res
         const int i = NG + (int)(t % G.nx); t /= G.nx;
         const int j = NG + (int)(t % G.ny);
         const int k = NG + (int)(t / G.ny);
-        const int64_t c = uidx(G, i, j, k);
-        double u[5];
-#pragma unroll
-        for (int q = 0; q < 5; ++q) u[q] = G.U[q * G.fs + c];
-        if (copy_un) {
-#pragma unroll
-            for (int q = 0; q < 5; ++q) G.Un[q * G.fs + c] = u[q];
-        }
-        // the split form floors with the same division wherever it floors
-        const bool fired = G.prec == 1 ? apply_floor<true>(u, G.rho_floor, G.P_floor, G.gamma)
-                                       : apply_floor<false>(u, G.rho_floor, G.P_floor, G.gamma);
-        if (fired) {
-#pragma unroll
-            for (int q = 0; q < 5; ++q) G.U[q * G.fs + c] = u[q];
-        }
+        floor_cell(G, uidx(G, i, j, k), copy_un);
     }
 }
 
@@ -1757,30 +1764,95 @@ __global__ __launch_bounds__(64) void k_prolong(const GridDev* __restrict__ grid
     }
 }
 
+__device__ __forceinline__ bool in_shell(const FmrDev& M, int axis, int p) {
+    return p <= M.slo[axis] || p >= M.shi[axis];
+}
+
 // U_c_interp = (1 - alpha) * U_c_n + alpha * U_c_np1 (fmr3d.jl:547-551) over
-// the parent cells the child's prolongation stencils read, once per fine
-// sub-cycle (alpha is fixed for its three stages).
+// the parent cells the child's ghost stencils read, once per fine sub-cycle
+// (alpha is fixed for its three stages): the x slabs read the transposed copy,
+// the others the plain one, none the inside of the box.
 __global__ void k_time_interp(const GridDev* __restrict__ grids, const FmrDev* __restrict__ fmr,
                               double alpha) {
     const FmrDev& M = *fmr;
     const GridDev& C = grids[M.parent];
-    const int nx = M.phi[0] - M.plo[0] + 1, ny = M.phi[1] - M.plo[1] + 1;
-    const int64_t total = (int64_t)nx * ny * (M.phi[2] - M.plo[2] + 1);
+    const int nx = M.phi[0] - M.plo[0] + 1, ny = M.phi[1] - M.plo[1] + 1, nz = M.phi[2] - M.plo[2] + 1;
+    const int64_t total = (int64_t)nx * ny * nz;
     const double oma = 1.0 - alpha;
     for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < total;
          e += (int64_t)gridDim.x * blockDim.x) {
         const int i = M.plo[0] + (int)(e % nx);
         const int64_t r = e / nx;
         const int j = M.plo[1] + (int)(r % ny), k = M.plo[2] + (int)(r / ny);
+        const bool xs = in_shell(M, 0, i), yz = in_shell(M, 1, j) || in_shell(M, 2, k);
+        if (!xs && !yz) continue;
         const int64_t o = uidx(C, i, j, k);
-        const int nz = M.phi[2] - M.plo[2] + 1;
         const int64_t ot = ((int64_t)(i - M.plo[0]) * nz + (k - M.plo[2])) * ny + (j - M.plo[1]);
 #pragma unroll
         for (int q = 0; q < 5; ++q) {
             const double v = oma * M.Ucn[q * C.fs + o] + alpha * M.Ucnp1[q * C.fs + o];
-            M.Uci[q * C.fs + o] = v;
-            M.Ucit[q * total + ot] = v;
+            if (yz) M.Uci[q * C.fs + o] = v;
+            if (xs) M.Ucit[q * total + ot] = v;
         }
+    }
+}
+
+// Start of a level's fused step: its ghost cells, which the stage-3 combination
+// reads after the prolongation has replaced them, are saved to Un (a child, own
+// != 0); so is what its child's ghost stencils read of the state at the start,
+// and the child's flux registers are cleared (a parent, fmr != null).  Copying
+// the whole state took 258 of 6270 us per root step of three levels from 192^3,
+// now 90.
+__global__ void k_level_begin(const GridDev* __restrict__ grids, int level, const FmrDev* __restrict__ fmr,
+                              int own) {
+    const GridDev& G = grids[level];
+    int64_t nb = 0, nr = 0;
+    int nx = 1, ny = 1;
+    if (fmr) {
+        nx = fmr->phi[0] - fmr->plo[0] + 1;
+        ny = fmr->phi[1] - fmr->plo[1] + 1;
+        nb = (int64_t)nx * ny * (fmr->phi[2] - fmr->plo[2] + 1);
+        nr = fmr->froff[6];
+    }
+    const int64_t ng = own ? ghost_count(G) : 0, total = ng + nb + nr;
+    for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < total;
+         e += (int64_t)gridDim.x * blockDim.x) {
+        if (e >= ng + nb) {
+            fmr->frc[e - ng - nb] = 0.0;
+            fmr->frf[e - ng - nb] = 0.0;
+            continue;
+        }
+        int i, j, k;
+        if (e < ng) {
+            ghost_decode(G, e, i, j, k);
+        } else {
+            const int64_t t = e - ng;
+            i = fmr->plo[0] + (int)(t % nx);
+            const int64_t r = t / nx;
+            j = fmr->plo[1] + (int)(r % ny);
+            k = fmr->plo[2] + (int)(r / ny);
+            if (!in_shell(*fmr, 0, i) && !in_shell(*fmr, 1, j) && !in_shell(*fmr, 2, k)) continue;
+        }
+        const int64_t c = uidx(G, i, j, k);
+#pragma unroll
+        for (int q = 0; q < 5; ++q) G.Un[q * G.fs + c] = G.U[q * G.fs + c];
+    }
+}
+
+// Floors on the cells of a parent that restriction and flux correction changed:
+// the child's box and one cell around it.  The others were floored by the last
+// stage, and a floored cell stays as it is under the floors.
+__global__ void k_floors_box(const GridDev* __restrict__ grids, const FmrDev* __restrict__ fmr) {
+    const FmrDev& M = *fmr;
+    const GridDev& G = grids[M.parent];
+    const int i0 = max(M.lo[0] - 1, 1), j0 = max(M.lo[1] - 1, 1), k0 = max(M.lo[2] - 1, 1);
+    const int nx = min(M.hi[0] + 1, G.nx) - i0 + 1, ny = min(M.hi[1] + 1, G.ny) - j0 + 1;
+    const int64_t total = (int64_t)nx * ny * (min(M.hi[2] + 1, G.nz) - k0 + 1);
+    for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < total;
+         e += (int64_t)gridDim.x * blockDim.x) {
+        const int64_t r = e / nx;
+        floor_cell(G, uidx(G, NG - 1 + i0 + (int)(e % nx), NG - 1 + j0 + (int)(r % ny), NG - 1 + k0 + (int)(r / ny)),
+                   false);
     }
 }
 
@@ -1864,16 +1936,6 @@ __device__ __forceinline__ void face_dims(const FmrDev& M, int face, int& n1, in
     if (face < 2)      { n1 = njc; n2 = nkc; }
     else if (face < 4) { n1 = nic; n2 = nkc; }
     else               { n1 = nic; n2 = njc; }
-}
-
-__global__ void k_fr_zero(const FmrDev* __restrict__ fmr) {
-    const FmrDev& M = *fmr;
-    const int64_t n = M.froff[6];
-    for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < n;
-         e += (int64_t)gridDim.x * blockDim.x) {
-        M.frc[e] = 0.0;
-        M.frf[e] = 0.0;
-    }
 }
 
 template <typename T>
@@ -2379,8 +2441,25 @@ hipError_t launch_scale(const LaunchCtx& L, double* a, int64_t n, double s) {
     return hipGetLastError();
 }
 
-hipError_t launch_fr_zero(const LaunchCtx& L, const FmrDev* fmr, int64_t total) {
-    hipLaunchKernelGGL(k_fr_zero, dim3(flat_blocks(total, L.cus)), dim3(256), 0, L.stream, fmr);
+hipError_t launch_level_begin(const LaunchCtx& L, const GridDev* grids, int level, const GridDev& h,
+                              const FmrDev* fmr, const FmrDev* hf, int own) {
+    const int64_t ghosts = 2LL * NG * ((int64_t)h.Ny * h.Nz + (int64_t)h.nx * h.Nz + (int64_t)h.nx * h.ny);
+    int64_t total = own ? ghosts : 0;
+    if (fmr) {
+        int64_t box = 1;
+        for (int a = 0; a < 3; ++a) box *= hf->phi[a] - hf->plo[a] + 1;
+        total += box + hf->froff[6];
+    }
+    if (total <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_level_begin, dim3(flat_blocks(total, L.cus)), dim3(256), 0, L.stream, grids, level,
+                       fmr, own);
+    return hipGetLastError();
+}
+
+hipError_t launch_floors_box(const LaunchCtx& L, const GridDev* grids, const FmrDev* fmr, const FmrDev& hf) {
+    int64_t box = 1;
+    for (int a = 0; a < 3; ++a) box *= hf.hi[a] - hf.lo[a] + 3;
+    hipLaunchKernelGGL(k_floors_box, dim3(flat_blocks(box, L.cus)), dim3(256), 0, L.stream, grids, fmr);
     return hipGetLastError();
 }
 

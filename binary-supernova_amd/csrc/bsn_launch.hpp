@@ -84,7 +84,9 @@ hipError_t launch_restrict(const LaunchCtx& L, const GridDev* grids, const FmrDe
 hipError_t launch_prolong_scalar(const LaunchCtx& L, const double* phc, const int nc[3], double* phf,
                                  const int nf[3], const int lo[3], int ratio);
 hipError_t launch_scale(const LaunchCtx& L, double* a, int64_t n, double s);
-hipError_t launch_fr_zero(const LaunchCtx& L, const FmrDev* fmr, int64_t total);
+hipError_t launch_level_begin(const LaunchCtx& L, const GridDev* grids, int level, const GridDev& h,
+                              const FmrDev* fmr, const FmrDev* hf, int own);
+hipError_t launch_floors_box(const LaunchCtx& L, const GridDev* grids, const FmrDev* fmr, const FmrDev& hf);
 hipError_t launch_fr_coarse(const LaunchCtx& L, int prec, const GridDev* grids, const FmrDev* fmr,
                             int64_t nelem, double weight);
 hipError_t launch_fr_fine(const LaunchCtx& L, int prec, const GridDev* grids, const FmrDev* fmr,
