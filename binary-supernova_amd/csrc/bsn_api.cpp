@@ -105,6 +105,13 @@ struct Plan {
     Tile* d_ft[3] = {nullptr, nullptr, nullptr};
     int nft[3] = {0, 0, 0};
     Tile* d_ut = nullptr;
+    // small grids (plan_small): one list for the three sweeps, one of single-cell
+    // update tiles; shapes set by the caller go back to the separate kernels
+    bool small = false;
+    Tile* d_sw = nullptr;
+    int nsw[3] = {0, 0, 0};
+    Tile* d_ut1 = nullptr;
+    int nut1 = 0;
     int nut = 0;
     // out-of-place step: descriptor tables of stages 1..3 and z-update tiles
     GridDev* d_st[3] = {nullptr, nullptr, nullptr};
@@ -379,11 +386,11 @@ static std::vector<Tile> flux_tiles(const std::vector<GridDev>& G, int dir, int 
     return t;
 }
 
-static std::vector<Tile> update_tiles(const std::vector<GridDev>& G) {
+static std::vector<Tile> update_tiles(const std::vector<GridDev>& G, int kz = UPDATE_KZ) {
     std::vector<Tile> t;
     for (int g = 0; g < (int)G.size(); ++g) {
         const GridDev& d = G[g];
-        for (int k0 = 0; k0 < d.nz; k0 += UPDATE_KZ)
+        for (int k0 = 0; k0 < d.nz; k0 += kz)
             for (int j0 = 0; j0 < d.ny; j0 += 4)
                 for (int i0 = 0; i0 < d.nx; i0 += 64) t.push_back({g, i0, j0, k0});
     }
@@ -514,6 +521,36 @@ static int plan_set_zshape(Plan& P, int shape) {
     return BSN_OK;
 }
 
+// Small grids step with all three sweeps in one launch and an update of one cell
+// per thread: their kernels take the latency of a launch and of one interface,
+// whatever their size.  Per device-dt step, one launch per kernel against merged:
+//   FP64   8^3 121 -> 78 us, 32^3 130 -> 95, 48^3 178 -> 151, 56^3 216 -> 205,
+//          64^3 266 -> 261, 80^3 391 -> 490;
+//   split  8^3 90 -> 63, 32^3 95 -> 73, 48^3 123 -> 103, 56^3 150 -> 139,
+//          64^3 162 -> 178.
+// A workgroup holds one tile and does not walk on to the next, so beyond a few
+// tiles per CU the starts and the z fluxes' way through memory cost more than
+// the launches: at 5 per CU (56^3 has 4.4 to 4.7, 64^3 5.9) merged still wins.
+static const int SMALL_TILES = 5;
+static int plan_small(Plan& P, const std::vector<GridDev>& G) {
+    const int64_t most = (int64_t)SMALL_TILES * P.ctx->cus;
+    P.small = false;
+    if (P.atotal > 256 * most) return BSN_OK;       // more x interfaces alone
+    std::vector<Tile> t;
+    for (int d = 0; d < 3; ++d) {
+        const auto l = flux_tiles(G, d, d == 0 ? 0 : FLUX_WALK_SHAPE0 + 2, P.ctx->cus, P.ctx->cus);
+        P.nsw[d] = (int)l.size();
+        t.insert(t.end(), l.begin(), l.end());
+    }
+    if ((int64_t)t.size() > most) return BSN_OK;
+    CHK(upload_vec(&P.d_sw, t));
+    const auto u = update_tiles(G, 1);
+    CHK(upload_vec(&P.d_ut1, u));
+    P.nut1 = (int)u.size();
+    P.small = true;
+    return BSN_OK;
+}
+
 static int plan_build(Plan& P) {
     HIPCHK(hipSetDevice(P.ctx->device));
     CHK(plan_refresh(P));
@@ -533,7 +570,7 @@ static int plan_build(Plan& P) {
     CHK(upload_vec(&P.d_aoff, ao));
     P.gtotal = go.back();
     P.atotal = ao.back();
-    return BSN_OK;
+    return plan_small(P, G);
 }
 
 static void plan_free(Plan* P) {
@@ -544,6 +581,8 @@ static void plan_free(Plan* P) {
     (void)hipFree(P->d_grids);
     for (int d = 0; d < 3; ++d) (void)hipFree(P->d_ft[d]);
     (void)hipFree(P->d_ut);
+    (void)hipFree(P->d_sw);
+    (void)hipFree(P->d_ut1);
     for (int s = 0; s < 3; ++s) (void)hipFree(P->d_st[s]);
     (void)hipFree(P->d_zt);
     (void)hipFree(P->d_goff);
@@ -590,6 +629,10 @@ static void prof_mark(Plan& P, int kind) {
 static int plan_fluxes(Plan& P, const GridDev* table = nullptr, int ndirs = 3) {
     const LaunchCtx L = P.ctx->L();
     if (!table) table = P.d_grids;
+    if (P.small && !P.prof) {
+        HIPCHK(launch_sweeps(L, P.prec, table, P.d_sw, P.nsw));
+        return BSN_OK;
+    }
     for (int d = 0; d < ndirs; ++d) {
         prof_mark(P, d);
         HIPCHK(launch_flux(L, d, P.prec, P.kshape[d], table, P.d_ft[d], P.nft[d], 0));
@@ -598,9 +641,27 @@ static int plan_fluxes(Plan& P, const GridDev* table = nullptr, int ndirs = 3) {
     return BSN_OK;
 }
 
-static int plan_update(Plan& P, int stage, int do_cfl, double* dU_out = nullptr) {
+// Profiling times the kernels one by one, so a profiled step of small grids takes
+// the separate ones.
+static bool small_step(const Plan& P) { return P.small && !P.prof; }
+
+static int plan_update(Plan& P, int stage, int do_cfl, double* dU_out = nullptr,
+                       const GridDev* table = nullptr) {
+    if (!table) table = P.d_grids;
     prof_mark(P, 3);
-    HIPCHK(launch_update(P.ctx->L(), P.prec, P.d_grids, P.d_ut, P.nut, stage, do_cfl, dU_out));
+    if (small_step(P)) HIPCHK(launch_update(P.ctx->L(), P.prec, 1, table, P.d_ut1, P.nut1, stage, do_cfl, dU_out));
+    else HIPCHK(launch_update(P.ctx->L(), P.prec, UPDATE_KZ, table, P.d_ut, P.nut, stage, do_cfl, dU_out));
+    prof_mark(P, 9);
+    return BSN_OK;
+}
+
+// The rest of a stage of the out-of-place step, after plan_fluxes(P, table, 2): the
+// z sweep fused with the update, or, small grids, whose z fluxes are there
+// already, the update alone.  Same bits.
+static int stage_update(Plan& P, const GridDev* table, int stage, int do_cfl) {
+    if (small_step(P)) return plan_update(P, stage, do_cfl, nullptr, table);
+    prof_mark(P, 3);
+    HIPCHK(launch_zupdate(P.ctx->L(), P.prec, P.zshape, table, P.d_zt, P.nzt, stage, do_cfl));
     prof_mark(P, 9);
     return BSN_OK;
 }
@@ -639,9 +700,7 @@ static int plan_step(Plan& P, int fused_cfl) {
             in.U = s == 1 ? g->h.U : s == 2 ? g->h.Un : g->d_work;
             HIPCHK(poisson_solve_state(*g->pois, in, s == 1, g->d_phi, L.stream));
         }
-        prof_mark(P, 3);
-        HIPCHK(launch_zupdate(L, P.prec, P.zshape, T, P.d_zt, P.nzt, s, fused_cfl && s == 3));
-        prof_mark(P, 9);
+        CHK(stage_update(P, T, s, fused_cfl && s == 3));
     }
     CHK(plan_ghost_combine(P, 3, P.d_st[2]));
     return BSN_OK;
@@ -674,7 +733,8 @@ static int plan_cfl(Plan& P, double cfl, double t_end) {
         HIPCHK(launch_set_scal(L, g->h.scal, SCAL_CFL, cfl));
         HIPCHK(launch_set_scal(L, g->h.scal, SCAL_TEND, t_end));
     }
-    HIPCHK(launch_cfl(L, P.d_grids, P.d_ut, P.nut));
+    if (P.small) HIPCHK(launch_cfl(L, 1, P.d_grids, P.d_ut1, P.nut1));
+    else         HIPCHK(launch_cfl(L, UPDATE_KZ, P.d_grids, P.d_ut, P.nut));
     return BSN_OK;
 }
 
@@ -1587,6 +1647,7 @@ extern "C" int bsn_batch_set_shapes(bsn_batch* b, int sx, int sy, int sz) {
         if (s[d] < 0 || s[d] >= flux_shape_count(d)) return set_err(BSN_ERR_ARG, "shape %d", s[d]);
     HIPCHK(hipSetDevice(b->plan->ctx->device));
     for (int d = 0; d < 3; ++d) CHK(plan_set_shape(*b->plan, d, s[d]));
+    b->plan->small = false;
     return BSN_OK;
 }
 
@@ -1594,7 +1655,9 @@ extern "C" int bsn_batch_set_update_shape(bsn_batch* b, int shape) {
     if (!b) return set_err(BSN_ERR_ARG, "NULL batch");
     if (shape < 0 || shape >= zupdate_shape_count()) return set_err(BSN_ERR_ARG, "shape %d", shape);
     HIPCHK(hipSetDevice(b->plan->ctx->device));
-    return plan_set_zshape(*b->plan, shape);
+    CHK(plan_set_zshape(*b->plan, shape));
+    b->plan->small = false;
+    return BSN_OK;
 }
 
 extern "C" int bsn_batch_get_shapes(bsn_batch* b, int shapes[4]) {
@@ -2096,9 +2159,7 @@ static int fmr_advance(bsn_fmr* m, int l) {
         for (int s = 1; s <= 3; ++s) {
             const GridDev* T = m->d_fst[4 * l + s - 1];
             CHK(plan_fluxes(P, T, 2));
-            prof_mark(P, 3);
-            HIPCHK(launch_zupdate(L, P.prec, P.zshape, T, P.d_zt, P.nzt, s, 0));
-            prof_mark(P, 9);
+            CHK(stage_update(P, T, s, 0));
             if (child) HIPCHK(launch_fr_coarse(L, P.prec, m->d_all, m->d_f + l, m->hf[l].froff[6] / 5, RK_W[s - 1]));
             if (l > 0) HIPCHK(launch_fr_fine(L, P.prec, m->d_all, m->d_f + (l - 1), m->hf[l - 1].froff[6] / 5, RK_W[s - 1]));
         }

@@ -378,9 +378,10 @@ __device__ __forceinline__ void store_face(const GridDev& G, const T (&F)[5], in
     for (int q = 0; q < 5; ++q) __builtin_nontemporal_store(F[q], &Fp[q * G.ffs[DIR] + o]);
 }
 
-template <int DIR, typename T, int W, int H, bool FLAT = false>
-__global__ __launch_bounds__(W * H, (DIR == 0 && W == 64 && H == 4 && sizeof(T) == 4) ? 6 : 1) void k_flux(const GridDev* __restrict__ grids,
-                                                 const Tile* __restrict__ tiles, int ntiles) {
+// tiles t0 .. t1 - 1 of a list
+template <int DIR, typename T, int W, int H, bool FLAT>
+__device__ __forceinline__ void flux_tiles(const GridDev* __restrict__ grids, const Tile* __restrict__ tiles,
+                                           int t0, int t1) {
     constexpr int NT = W * H;
     constexpr bool FAST = sizeof(T) == 4;        // split form
     constexpr int SA = DIR == 0 ? H : H + 5;     // LDS rows
@@ -397,8 +398,6 @@ __global__ __launch_bounds__(W * H, (DIR == 0 && W == 64 && H == 4 && sizeof(T) 
     constexpr int LW = 64 + 5 * XFLAT_ROWS;      // staged cells of a wave, FLAT
     __shared__ T lds[5][FLAT ? H : SA][FLAT ? LW : SB];
     const int tid = threadIdx.x;
-    int t0, t1;
-    chunk(ntiles, t0, t1);
     typename Prec<T>::Carry nc[5];               // unused: no indicators are carried between tiles
     for (int t = t0; t < t1; ++t) {
         const Tile tl = tiles[t];
@@ -661,6 +660,14 @@ __global__ __launch_bounds__(W * H, (DIR == 0 && W == 64 && H == 4 && sizeof(T) 
     }
 }
 
+template <int DIR, typename T, int W, int H, bool FLAT = false>
+__global__ __launch_bounds__(W * H, (DIR == 0 && W == 64 && H == 4 && sizeof(T) == 4) ? 6 : 1) void k_flux(const GridDev* __restrict__ grids,
+                                                 const Tile* __restrict__ tiles, int ntiles) {
+    int t0, t1;
+    chunk(ntiles, t0, t1);
+    flux_tiles<DIR, T, W, H, FLAT>(grids, tiles, t0, t1);
+}
+
 // x interface fluxes as short register walks.  Tile (g, f0, j0, k | n): a
 // block of four waves stages rows j0 .. j0+3 of plane k, cells f0 .. f0+n+4
 // (padded x), in LDS; lane l of wave w walks row j0+w through its share of
@@ -826,11 +833,9 @@ __global__ __launch_bounds__(256) void k_fxwalk(const GridDev* __restrict__ grid
 // The FP64 form carries them too, with their reciprocals, at 255 VGPRs, 2 waves
 // per SIMD.
 template <int DIR, typename T>
-__global__ __launch_bounds__(256, sizeof(T) == 4 ? 4 : 2) void k_fwalk(const GridDev* __restrict__ grids,
-                                               const Tile* __restrict__ tiles, int ntiles) {
+__device__ __forceinline__ void walk_tiles(const GridDev* __restrict__ grids, const Tile* __restrict__ tiles,
+                                           int t0, int t1) {
     constexpr bool FAST = sizeof(T) == 4;        // split form
-    int t0, t1;
-    chunk(ntiles, t0, t1);
     for (int t = t0; t < t1; ++t) {
         const Tile tl = tiles[t];
         const GridDev& G = grids[tl.g];
@@ -917,6 +922,28 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 4 : 2) void k_fwalk(const Gri
         }
         for (; f < fend; ++f) step(f);
     }
+}
+
+template <int DIR, typename T>
+__global__ __launch_bounds__(256, sizeof(T) == 4 ? 4 : 2) void k_fwalk(const GridDev* __restrict__ grids,
+                                               const Tile* __restrict__ tiles, int ntiles) {
+    int t0, t1;
+    chunk(ntiles, t0, t1);
+    walk_tiles<DIR, T>(grids, tiles, t0, t1);
+}
+
+// All three sweeps of small grids in one launch: the list holds nx x tiles (64 x 4
+// and flat), then ny y runs and the z runs, one per workgroup.  Such a sweep
+// leaves most of the chip idle and takes the latency of its launch and of one
+// interface, which this way is paid once (plan_small in bsn_api.cpp has the times).
+template <typename T>
+__global__ __launch_bounds__(256, sizeof(T) == 4 ? 4 : 2) void k_sweeps(const GridDev* __restrict__ grids,
+                                                                        const Tile* __restrict__ tiles, int nx,
+                                                                        int ny) {
+    const int b = (int)blockIdx.x;
+    if (b < nx)           flux_tiles<0, T, 64, 4, true>(grids, tiles, b, b + 1);
+    else if (b < nx + ny) walk_tiles<1, T>(grids, tiles, b, b + 1);
+    else                  walk_tiles<2, T>(grids, tiles, b, b + 1);
 }
 
 // ---------------------------------------------------------------------------
@@ -2181,20 +2208,32 @@ hipError_t launch_flux(const LaunchCtx& L, int dir, int prec, int shape, const G
     return launch_flux_shape<2, float>(L, shape, grids, tiles, ntiles, max_wg);
 }
 
-hipError_t launch_update(const LaunchCtx& L, int prec, const GridDev* grids, const Tile* tiles,
+template <typename T, int KZ>
+static hipError_t launch_update_t(const LaunchCtx& L, const GridDev* grids, const Tile* tiles, int ntiles,
+                                  int stage, int do_cfl, double* dU_out) {
+    const int g = KZ == 1 ? ntiles : occupancy_grid((const void*)&k_update<T, KZ>, 256, 0, ntiles, L.cus);
+    hipLaunchKernelGGL((k_update<T, KZ>), dim3(g), dim3(256), 0, L.stream, grids, tiles, ntiles, stage, do_cfl,
+                       dU_out);
+    return hipGetLastError();
+}
+
+hipError_t launch_update(const LaunchCtx& L, int prec, int kz, const GridDev* grids, const Tile* tiles,
                          int ntiles, int stage, int do_cfl, double* dU_out) {
     if (ntiles <= 0) return hipSuccess;
-    if (prec == 0) {
-        const void* fn = (const void*)&k_update<double, UPDATE_KZ>;
-        const int g = occupancy_grid(fn, 256, 0, ntiles, L.cus);
-        hipLaunchKernelGGL((k_update<double, UPDATE_KZ>), dim3(g), dim3(256), 0, L.stream, grids,
-                           tiles, ntiles, stage, do_cfl, dU_out);
-    } else {
-        const void* fn = (const void*)&k_update<float, UPDATE_KZ>;
-        const int g = occupancy_grid(fn, 256, 0, ntiles, L.cus);
-        hipLaunchKernelGGL((k_update<float, UPDATE_KZ>), dim3(g), dim3(256), 0, L.stream, grids,
-                           tiles, ntiles, stage, do_cfl, dU_out);
-    }
+    if (kz == 1)
+        return prec == 0 ? launch_update_t<double, 1>(L, grids, tiles, ntiles, stage, do_cfl, dU_out)
+                         : launch_update_t<float, 1>(L, grids, tiles, ntiles, stage, do_cfl, dU_out);
+    return prec == 0 ? launch_update_t<double, UPDATE_KZ>(L, grids, tiles, ntiles, stage, do_cfl, dU_out)
+                     : launch_update_t<float, UPDATE_KZ>(L, grids, tiles, ntiles, stage, do_cfl, dU_out);
+}
+
+hipError_t launch_sweeps(const LaunchCtx& L, int prec, const GridDev* grids, const Tile* tiles, const int n[3]) {
+    const int total = n[0] + n[1] + n[2];
+    if (total <= 0) return hipSuccess;
+    if (prec == 0)
+        hipLaunchKernelGGL(k_sweeps<double>, dim3(total), dim3(256), 0, L.stream, grids, tiles, n[0], n[1]);
+    else
+        hipLaunchKernelGGL(k_sweeps<float>, dim3(total), dim3(256), 0, L.stream, grids, tiles, n[0], n[1]);
     return hipGetLastError();
 }
 
@@ -2266,11 +2305,14 @@ hipError_t launch_zupdate(const LaunchCtx& L, int prec, int shape, const GridDev
     return launch_zupdate_p<float>(L, shape, grids, tiles, ntiles, stage, do_cfl);
 }
 
-hipError_t launch_cfl(const LaunchCtx& L, const GridDev* grids, const Tile* tiles, int ntiles) {
+hipError_t launch_cfl(const LaunchCtx& L, int kz, const GridDev* grids, const Tile* tiles, int ntiles) {
     if (ntiles <= 0) return hipSuccess;
-    const void* fn = (const void*)&k_cfl<UPDATE_KZ>;
-    const int g = occupancy_grid(fn, 256, 0, ntiles, L.cus);
-    hipLaunchKernelGGL((k_cfl<UPDATE_KZ>), dim3(g), dim3(256), 0, L.stream, grids, tiles, ntiles);
+    if (kz == 1) {
+        hipLaunchKernelGGL(k_cfl<1>, dim3(ntiles), dim3(256), 0, L.stream, grids, tiles, ntiles);
+    } else {
+        const int g = occupancy_grid((const void*)&k_cfl<UPDATE_KZ>, 256, 0, ntiles, L.cus);
+        hipLaunchKernelGGL(k_cfl<UPDATE_KZ>, dim3(g), dim3(256), 0, L.stream, grids, tiles, ntiles);
+    }
     return hipGetLastError();
 }
 

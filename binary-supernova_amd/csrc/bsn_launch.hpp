@@ -29,9 +29,13 @@ int flux_slots(int dir, int prec, int shape, int cus);
 
 hipError_t launch_flux(const LaunchCtx& L, int dir, int prec, int shape, const GridDev* grids,
                        const Tile* tiles, int ntiles, int max_wg);
-hipError_t launch_update(const LaunchCtx& L, int prec, const GridDev* grids, const Tile* tiles,
+// kz: cells per thread of the tile list, 1 or UPDATE_KZ
+hipError_t launch_update(const LaunchCtx& L, int prec, int kz, const GridDev* grids, const Tile* tiles,
                          int ntiles, int stage, int do_cfl, double* dU_out);
-hipError_t launch_cfl(const LaunchCtx& L, const GridDev* grids, const Tile* tiles, int ntiles);
+// The three sweeps in one launch: tiles holds n[0] x tiles of shape 0, n[1] y runs
+// and n[2] z runs.
+hipError_t launch_sweeps(const LaunchCtx& L, int prec, const GridDev* grids, const Tile* tiles, const int n[3]);
+hipError_t launch_cfl(const LaunchCtx& L, int kz, const GridDev* grids, const Tile* tiles, int ntiles);
 int zupdate_shape_count();
 int zupdate_seg(int shape);
 int zupdate_slots(int prec, int shape, int cus);
