@@ -17,6 +17,7 @@
 #include <cstdio>
 #include <cmath>
 #include <cstring>
+#include <mutex>
 #include <numeric>
 #include <queue>
 #include <string>
@@ -61,13 +62,172 @@ static inline int64_t round_up(int64_t a, int64_t m) { return (a + m - 1) / m * 
 // ---------------------------------------------------------------------------
 // Objects
 
+// Pinned memory that host arrays pass through, one per context (HostXfer).
+struct HostPipe {
+    static const int SLOTS = 4;
+    static const size_t SLOT = 2 << 20;
+    std::mutex mu;               // held for a transfer
+    char* buf = nullptr;         // SLOTS slots, then a few scalars that kernels write
+    hipEvent_t ev[SLOTS] = {};   // after the last copy from or to a slot
+    bool busy[SLOTS] = {};       // that copy may still be running
+    int next = 0;
+    double* scalars() const { return (double*)(buf + SLOTS * SLOT); }
+};
+
 struct bsn_ctx {
+    HostPipe pipe;
     int device = 0;
     hipStream_t stream = nullptr;
     int cus = 1;
     double* totals_scratch = nullptr;   // device address of the fixed totals scratch
     char name[256] = {0};
     LaunchCtx L() const { return LaunchCtx{stream, cus}; }
+};
+
+// Copies between host arrays and the device on the context's stream, a slot of
+// pinned memory at a time: the CPU fills or empties one while the others are in
+// flight.  The link moves 13.7 MB in 250 us and 256 kB in 13; left to the runtime,
+// pageable memory takes 800 us to the host, and 110 for the 256 kB either way.  Here
+// one thread's copying (28 GB/s from memory, 62 to it) sets the pace: a host loop
+// on numpy arrays takes 0.19 ms per step at 8^3 (0.50 by the runtime's copies), 0.60
+// at 32^3 (0.82), 2.1 at 64^3 (2.5).  Three helper threads doubled the copying, but
+// their start cost a 4 MB array more (40^3 1.43 ms against 0.93) than they gave a
+// 14 MB one.  Memory that is pinned already is copied directly.
+//
+// The object holds the pipe for as long as it lives; data has arrived in host
+// arrays after flush().
+class HostXfer {
+    bsn_ctx* c;
+    std::lock_guard<std::mutex> lk;
+    struct Out { char* dst; size_t n; int slot; } q[HostPipe::SLOTS];    // not taken yet, oldest first
+    int qn = 0;
+
+    // the runtime's own copy from pageable memory is as fast beyond this (139 us for
+    // 4.2 MB; 367 for 1 MB, here 45)
+    static const size_t DIRECT_FROM = 3 << 20;
+
+    char* mem(int s) const { return c->pipe.buf + s * HostPipe::SLOT; }
+    // a copy has its launch and its event to pay (14 us): parts of 1 MB, 2 of
+    // larger arrays
+    static size_t part(size_t n) { return n > (8 << 20) ? HostPipe::SLOT : HostPipe::SLOT / 2; }
+
+    int ready() {
+        HostPipe& p = c->pipe;
+        if (p.buf) return BSN_OK;
+        for (auto& e : p.ev)
+            if (!e) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+        HIPCHK(hipHostMalloc((void**)&p.buf, HostPipe::SLOTS * HostPipe::SLOT + 4096, hipHostMallocDefault));
+        return BSN_OK;
+    }
+    int take() {
+        HostPipe& p = c->pipe;
+        const Out o = q[0];
+        HIPCHK(hipEventSynchronize(p.ev[o.slot]));
+        p.busy[o.slot] = false;
+        memcpy(o.dst, mem(o.slot), o.n);
+        for (int i = 1; i < qn; ++i) q[i - 1] = q[i];
+        --qn;
+        return BSN_OK;
+    }
+    // the next slot, with nothing in it or on its way
+    int slot(int& s) {
+        HostPipe& p = c->pipe;
+        s = p.next;
+        p.next = (s + 1) % HostPipe::SLOTS;
+        while (qn > 0 && q[0].slot == s) CHK(take());
+        if (p.busy[s]) HIPCHK(hipEventSynchronize(p.ev[s]));
+        p.busy[s] = false;
+        return BSN_OK;
+    }
+    int sent(int s) {
+        HIPCHK(hipEventRecord(c->pipe.ev[s], c->stream));
+        c->pipe.busy[s] = true;
+        return BSN_OK;
+    }
+    static bool pageable(const void* p) {
+        hipPointerAttribute_t a;
+        if (hipPointerGetAttributes(&a, p) == hipSuccess) return a.type == hipMemoryTypeUnregistered;
+        (void)hipGetLastError();
+        return true;
+    }
+
+public:
+    explicit HostXfer(bsn_ctx* ctx) : c(ctx), lk(ctx->pipe.mu) {}
+    ~HostXfer() {
+        // after an error: nothing may still be on its way to a slot
+        if (qn > 0) (void)hipStreamSynchronize(c->stream);
+    }
+    HostXfer(const HostXfer&) = delete;
+    HostXfer& operator=(const HostXfer&) = delete;
+
+    // on return src has been read
+    int in(void* dst, const void* src, size_t n) {
+        if (n > DIRECT_FROM || !pageable(src)) {
+            HIPCHK(hipMemcpyAsync(dst, src, n, hipMemcpyHostToDevice, c->stream));
+            return BSN_OK;
+        }
+        CHK(ready());
+        for (size_t o = 0, m = part(n); o < n; o += m) {
+            const size_t k = std::min(n - o, m);
+            int s;
+            CHK(slot(s));
+            memcpy(mem(s), (const char*)src + o, k);
+            HIPCHK(hipMemcpyAsync((char*)dst + o, mem(s), k, hipMemcpyHostToDevice, c->stream));
+            CHK(sent(s));
+        }
+        return BSN_OK;
+    }
+    int out(void* dst, const void* src, size_t n) {
+        if (!pageable(dst)) {
+            HIPCHK(hipMemcpyAsync(dst, src, n, hipMemcpyDeviceToHost, c->stream));
+            return BSN_OK;
+        }
+        CHK(ready());
+        for (size_t o = 0, m = part(n); o < n; o += m) {
+            const size_t k = std::min(n - o, m);
+            int s;
+            CHK(slot(s));
+            HIPCHK(hipMemcpyAsync(mem(s), (const char*)src + o, k, hipMemcpyDeviceToHost, c->stream));
+            CHK(sent(s));
+            q[qn++] = {(char*)dst + o, k, s};
+        }
+        return BSN_OK;
+    }
+    int flush() {
+        while (qn > 0) CHK(take());
+        return BSN_OK;
+    }
+    // host memory that a kernel can write; read it after the stream is done
+    int scalars(double*& p) {
+        CHK(ready());
+        p = c->pipe.scalars();
+        return BSN_OK;
+    }
+};
+
+// A device table of descriptors with the host's copy of what it holds: uploaded,
+// in the stream's order, only when that has changed.  (A refresh of a two-level
+// hierarchy was 17 synchronous copies.)
+struct DescTable {
+    GridDev* d = nullptr;
+    std::vector<GridDev> held;
+
+    int set(bsn_ctx* c, const std::vector<GridDev>& v) {
+        const size_t bytes = v.size() * sizeof(GridDev);
+        if (d && held.size() == v.size() && memcmp(held.data(), v.data(), bytes) == 0) return BSN_OK;
+        if (held.size() != v.size()) {
+            if (d) HIPCHK(hipFree(d));
+            d = nullptr;
+            held.clear();
+            HIPCHK(hipMalloc((void**)&d, bytes));
+        }
+        held.clear();
+        HostXfer x(c);
+        CHK(x.in(d, v.data(), bytes));
+        held = v;
+        return BSN_OK;
+    }
+    void free() { (void)hipFree(d); d = nullptr; held.clear(); }
 };
 
 struct Plan;
@@ -99,6 +259,7 @@ struct Plan {
     bsn_ctx* ctx = nullptr;
     std::vector<bsn_grid*> grids;
     int prec = 0;
+    DescTable desc;              // d_grids, then d_st[0..2]
     GridDev* d_grids = nullptr;
     int shape[3] = {0, 0, 0};
     int kshape[3] = {0, 0, 0};   // as launch_flux takes it (FLUX_XFLAT)
@@ -147,7 +308,8 @@ struct bsn_fmr {
     hipGraphExec_t gexec = nullptr;
     hipGraph_t graph = nullptr;
     int inplace = 0;                 // 1: levels step in place with all fluxes materialised
-    std::vector<GridDev*> d_fst;     // per level, the three stage tables of the fused step
+    DescTable all;                   // d_all, then d_fst
+    GridDev* d_fst = nullptr;        // per level, the four stage tables of the fused step
     // self-gravity (fmr3d_step! with self_gravity = true, src/fmr3d.jl:451-473):
     // the frozen per-level phi of the root step, in buffers of its own
     int sg_on = 0;                   // bsn_fmr_run solves it every root step
@@ -487,27 +649,25 @@ static int ensure_work2(bsn_grid* g) {
 // never modified before stage 3.
 static int plan_refresh(Plan& P) {
     HIPCHK(hipSetDevice(P.ctx->device));
-    auto G = host_descs(P);
-    const size_t bytes = G.size() * sizeof(GridDev);
-    if (!P.d_grids) HIPCHK(hipMalloc((void**)&P.d_grids, bytes));
-    HIPCHK(hipMemcpy(P.d_grids, G.data(), bytes, hipMemcpyHostToDevice));
-    std::vector<GridDev> st[3];
-    for (size_t gi = 0; gi < G.size(); ++gi) {
+    const auto G = host_descs(P);
+    const size_t n = G.size();
+    std::vector<GridDev> t(4 * n);
+    for (size_t gi = 0; gi < n; ++gi) {
         bsn_grid* g = P.grids[gi];
         CHK(ensure_work(g));
         double* A = g->h.U;
         double* B = g->h.Un;
         double* C = g->d_work;
         GridDev d = G[gi];
+        t[gi] = d;
         d.Un = A;
-        d.lmode = 3; d.U = A; d.Uout = B; st[0].push_back(d);
-        d.lmode = 1; d.U = B; d.Uout = C; st[1].push_back(d);
-        d.lmode = 1; d.U = C; d.Uout = A; st[2].push_back(d);
+        d.lmode = 3; d.U = A; d.Uout = B; t[n + gi] = d;
+        d.lmode = 1; d.U = B; d.Uout = C; t[2 * n + gi] = d;
+        d.lmode = 1; d.U = C; d.Uout = A; t[3 * n + gi] = d;
     }
-    for (int s = 0; s < 3; ++s) {
-        if (!P.d_st[s]) HIPCHK(hipMalloc((void**)&P.d_st[s], bytes));
-        HIPCHK(hipMemcpy(P.d_st[s], st[s].data(), bytes, hipMemcpyHostToDevice));
-    }
+    CHK(P.desc.set(P.ctx, t));
+    P.d_grids = P.desc.d;
+    for (int s = 0; s < 3; ++s) P.d_st[s] = P.desc.d + (s + 1) * n;
     return BSN_OK;
 }
 
@@ -578,12 +738,11 @@ static void plan_free(Plan* P) {
     (void)hipSetDevice(P->ctx->device);
     graph_drop(P->gexec, P->graph);
     for (auto e : P->ev) (void)hipEventDestroy(e);
-    (void)hipFree(P->d_grids);
+    P->desc.free();
     for (int d = 0; d < 3; ++d) (void)hipFree(P->d_ft[d]);
     (void)hipFree(P->d_ut);
     (void)hipFree(P->d_sw);
     (void)hipFree(P->d_ut1);
-    for (int s = 0; s < 3; ++s) (void)hipFree(P->d_st[s]);
     (void)hipFree(P->d_zt);
     (void)hipFree(P->d_goff);
     (void)hipFree(P->d_aoff);
@@ -772,6 +931,9 @@ extern "C" int bsn_ctx_destroy(bsn_ctx* c) {
     if (!c) return BSN_OK;
     (void)hipSetDevice(c->device);
     (void)hipStreamSynchronize(c->stream);
+    for (auto& e : c->pipe.ev)
+        if (e) (void)hipEventDestroy(e);
+    if (c->pipe.buf) (void)hipHostFree(c->pipe.buf);
     (void)hipStreamDestroy(c->stream);
     delete c;
     return BSN_OK;
@@ -917,24 +1079,32 @@ static int import_ref(bsn_grid* g, const double* src, int where, double* dst) {
     const double* from = src;
     if (where == BSN_HOST) {
         CHK(ensure_stage(g, bytes));
-        HIPCHK(hipMemcpyAsync(g->d_stage, src, bytes, hipMemcpyHostToDevice, g->ctx->stream));
+        HostXfer x(g->ctx);
+        CHK(x.in(g->d_stage, src, bytes));
         from = g->d_stage;
     }
     HIPCHK(launch_aos_to_soa(L, g->h, from, dst));
     return BSN_OK;
 }
 
-static int export_ref(bsn_grid* g, const double* src, double* dst, int where) {
+// device buffer -> reference layout; a host array is filled when x is flushed
+static int export_ref(bsn_grid* g, const double* src, double* dst, int where, HostXfer& x) {
     const LaunchCtx L = g->ctx->L();
     const size_t bytes = (size_t)ref_count(g->h) * 8;
     if (where == BSN_HOST) {
         CHK(ensure_stage(g, bytes));
         HIPCHK(launch_soa_to_aos(L, g->h, src, g->d_stage));
-        HIPCHK(hipMemcpyAsync(dst, g->d_stage, bytes, hipMemcpyDeviceToHost, g->ctx->stream));
+        CHK(x.out(dst, g->d_stage, bytes));
     } else {
         HIPCHK(launch_soa_to_aos(L, g->h, src, dst));
     }
     return BSN_OK;
+}
+
+static int export_ref(bsn_grid* g, const double* src, double* dst, int where) {
+    HostXfer x(g->ctx);
+    CHK(export_ref(g, src, dst, where, x));
+    return x.flush();
 }
 
 extern "C" int bsn_grid_set_state(bsn_grid* g, const double* U, int where) {
@@ -965,7 +1135,8 @@ static int src_upload(bsn_grid* g) {
     const bool any = S.nbh > 0 || S.nsink > 0;
     if (any) {
         if (!g->d_src) HIPCHK(hipMalloc((void**)&g->d_src, sizeof(SrcDev)));
-        HIPCHK(hipMemcpy(g->d_src, &S, sizeof(SrcDev), hipMemcpyHostToDevice));
+        HostXfer x(g->ctx);
+        CHK(x.in(g->d_src, &S, sizeof(SrcDev)));
     }
     const SrcDev* want = any ? g->d_src : nullptr;
     if (g->h.src != want) {
@@ -1011,7 +1182,6 @@ extern "C" int bsn_grid_set_point_masses(bsn_grid* g, int n, const double* pos, 
     SrcDev S = g->hs;
     CHK(fill_masses(S, n, pos, mass, eps, x0, y0, z0));
     HIPCHK(hipSetDevice(g->ctx->device));
-    HIPCHK(hipStreamSynchronize(g->ctx->stream));
     g->hs = S;
     return src_upload(g);
 }
@@ -1023,7 +1193,6 @@ extern "C" int bsn_grid_set_sinks(bsn_grid* g, int n, const double* pos, const d
     SrcDev S = g->hs;
     CHK(fill_sinks(S, n, pos, vel, r_sink, t_sink, torque_free, rho_sink_min, x0, y0, z0));
     HIPCHK(hipSetDevice(g->ctx->device));
-    HIPCHK(hipStreamSynchronize(g->ctx->stream));
     g->hs = S;
     return src_upload(g);
 }
@@ -1110,11 +1279,11 @@ extern "C" int bsn_solve_poisson_isolated(bsn_grid* g, const double* rho, int wh
     if (!g->d_rho_in) HIPCHK(hipMalloc((void**)&g->d_rho_in, 2 * n * 8));
     const double* drho = where_rho == BSN_HOST ? g->d_rho_in : rho;
     double* dphi = where_phi == BSN_HOST ? g->d_rho_in + n : phi;
-    if (where_rho == BSN_HOST)
-        HIPCHK(hipMemcpyAsync(g->d_rho_in, rho, n * 8, hipMemcpyHostToDevice, g->ctx->stream));
+    HostXfer x(g->ctx);
+    if (where_rho == BSN_HOST) CHK(x.in(g->d_rho_in, rho, n * 8));
     HIPCHK(poisson_solve_array(*g->pois, drho, dphi, g->ctx->stream));
-    if (where_phi == BSN_HOST)
-        HIPCHK(hipMemcpyAsync(phi, dphi, n * 8, hipMemcpyDeviceToHost, g->ctx->stream));
+    if (where_phi == BSN_HOST) CHK(x.out(phi, dphi, n * 8));
+    CHK(x.flush());
     return sync_ctx(g->ctx);
 }
 
@@ -1152,7 +1321,12 @@ extern "C" int bsn_grid_set_phi(bsn_grid* g, const double* phi, int where) {
     }
     const size_t bytes = (size_t)g->h.nx * g->h.ny * g->h.nz * 8;
     if (!g->d_phi) HIPCHK(hipMalloc((void**)&g->d_phi, bytes));
-    HIPCHK(hipMemcpy(g->d_phi, phi, bytes, where == BSN_HOST ? hipMemcpyHostToDevice : hipMemcpyDeviceToDevice));
+    if (where == BSN_HOST) {
+        HostXfer x(g->ctx);
+        CHK(x.in(g->d_phi, phi, bytes));
+    } else {
+        HIPCHK(hipMemcpy(g->d_phi, phi, bytes, hipMemcpyDeviceToDevice));
+    }
     g->h.phi = g->d_phi;
     return grid_changed(g);
 }
@@ -1241,6 +1415,7 @@ extern "C" int bsn_euler3d_rhs(bsn_grid* g, double* dU, double* Fx, double* Fy, 
     CHK(plan_floors(P, 0));
     CHK(plan_fluxes(P));
     double* F[3] = {Fx, Fy, Fz};
+    HostXfer x(g->ctx);
     for (int d = 0; d < 3; ++d) {
         if (!F[d]) continue;
         const GridDev& h = g->h;
@@ -1248,8 +1423,7 @@ extern "C" int bsn_euler3d_rhs(bsn_grid* g, double* dU, double* Fx, double* Fy, 
         if (where == BSN_HOST) {
             CHK(ensure_stage(g, n * 8));
             HIPCHK(launch_flux_export(L, h, d, g->d_stage));
-            HIPCHK(hipMemcpyAsync(F[d], g->d_stage, n * 8, hipMemcpyDeviceToHost, g->ctx->stream));
-            HIPCHK(hipStreamSynchronize(g->ctx->stream));
+            CHK(x.out(F[d], g->d_stage, n * 8));
         } else {
             HIPCHK(launch_flux_export(L, h, d, F[d]));
         }
@@ -1258,8 +1432,9 @@ extern "C" int bsn_euler3d_rhs(bsn_grid* g, double* dU, double* Fx, double* Fy, 
         CHK(ensure_scratch(g));
         HIPCHK(launch_fill_u64(L, (uint64_t*)g->d_scratch, 5 * g->h.fs, 0));
         CHK(plan_update(P, 0, 0, g->d_scratch));
-        CHK(export_ref(g, g->d_scratch, dU, where));
+        CHK(export_ref(g, g->d_scratch, dU, where, x));
     }
+    CHK(x.flush());
     return sync_ctx(g->ctx);
 }
 
@@ -1282,9 +1457,13 @@ extern "C" int bsn_cfl_dt_3d(bsn_grid* g, double dx, double dy, double dz, doubl
     CHK(apply_params(g, dx, dy, dz, gamma, g->h.bc, g->h.rho_floor, g->h.P_floor));
     Plan& P = *g->plan;
     CHK(plan_cfl(P, cfl, 0.0));
-    HIPCHK(launch_dt(g->ctx->L(), P.d_grids, 1));
-    HIPCHK(hipMemcpyAsync(dt_out, &g->h.scal[SCAL_DT], 8, hipMemcpyDeviceToHost, g->ctx->stream));
-    return sync_ctx(g->ctx);
+    HostXfer x(g->ctx);
+    double* dt;
+    CHK(x.scalars(dt));
+    HIPCHK(launch_dt(g->ctx->L(), P.d_grids, 1, dt));
+    CHK(sync_ctx(g->ctx));
+    *dt_out = *dt;
+    return BSN_OK;
 }
 
 extern "C" int bsn_apply_sg_force(bsn_grid* g, double* dU, int where, double dx, double dy,
@@ -1325,7 +1504,9 @@ extern "C" int bsn_conserved_totals(bsn_grid* g, double dV, double out[5]) {
     const int nb = TOTALS_BLOCKS;
     if (!g->d_part) HIPCHK(hipMalloc((void**)&g->d_part, nb * 5 * 8));
     HIPCHK(launch_totals(g->ctx->L(), g->h, g->d_part, nb, dV, &g->h.scal[SCAL_TOT]));
-    HIPCHK(hipMemcpyAsync(out, &g->h.scal[SCAL_TOT], 5 * 8, hipMemcpyDeviceToHost, g->ctx->stream));
+    HostXfer x(g->ctx);
+    CHK(x.out(out, &g->h.scal[SCAL_TOT], 5 * 8));
+    CHK(x.flush());
     return sync_ctx(g->ctx);
 }
 
@@ -1374,9 +1555,11 @@ static int body_begin(bsn_grid* g, BodyQ& Q, double dx, double dy, double dz, do
 
 static int body_finish(bsn_grid* g, hipError_t e, double* host, int count) {
     if (e != hipSuccess) return set_err(BSN_ERR_HIP, "launch: %s", hipGetErrorString(e));
-    if (count > 0)
-        HIPCHK(hipMemcpyAsync(host, g->d_body + BODY_OUT, count * sizeof(double),
-                              hipMemcpyDeviceToHost, g->ctx->stream));
+    if (count > 0) {
+        HostXfer x(g->ctx);
+        CHK(x.out(host, g->d_body + BODY_OUT, count * sizeof(double)));
+        CHK(x.flush());
+    }
     return sync_ctx(g->ctx);
 }
 
@@ -1997,9 +2180,6 @@ extern "C" int bsn_fmr_create(bsn_ctx* ctx, int nlevels, bsn_grid* const* levels
         if (r != BSN_OK) return fail(r);
         m->plans.push_back(P);
     }
-    std::vector<GridDev> all;
-    for (auto* g : m->lev) all.push_back(g->h);
-    if (upload_vec(&m->d_all, all) != BSN_OK) return fail(BSN_ERR_HIP);
     for (int l = 0; l + 1 < nlevels; ++l) {
         FmrDev f{};
         f.parent = l;
@@ -2060,11 +2240,10 @@ extern "C" int bsn_fmr_destroy(bsn_fmr* m) {
     for (auto& f : m->hf) {
         (void)hipFree(f.frc); (void)hipFree(f.frf); (void)hipFree(f.Uci); (void)hipFree(f.Ucit);
     }
-    for (auto* t : m->d_fst) (void)hipFree(t);
     for (auto* p : m->d_sgphi) (void)hipFree(p);
     for (auto* g : m->lev) g->h.nzkeep = 0;
     (void)hipFree(m->d_f);
-    (void)hipFree(m->d_all);
+    m->all.free();
     delete m;
     return BSN_OK;
 }
@@ -2078,8 +2257,7 @@ extern "C" int bsn_fmr_destroy(bsn_fmr* m) {
 // under its boundary conditions on load; a child reads the ghost cells
 // prolonged into each stage input.  Stage 1 floors active cells on
 // load (the start-of-stage floors).
-static int fmr_stage_tables(bsn_fmr* m) {
-    if (m->d_fst.empty()) m->d_fst.assign(4 * m->nlev, nullptr);
+static int fmr_stage_tables(bsn_fmr* m, std::vector<GridDev>& t) {
     for (int l = 0; l < m->nlev; ++l) {
         bsn_grid* g = m->lev[l];
         CHK(ensure_work(g));
@@ -2093,21 +2271,19 @@ static int fmr_stage_tables(bsn_fmr* m) {
         st[2].lmode = map;     st[2].U = g->d_work2; st[2].Uout = g->h.U;
         st[3] = st[2];
         if (l > 0) st[3].Un = g->h.Un;
-        for (int s = 0; s < 4; ++s) {
-            GridDev*& t = m->d_fst[4 * l + s];
-            if (!t) HIPCHK(hipMalloc((void**)&t, sizeof(GridDev)));
-            HIPCHK(hipMemcpy(t, &st[s], sizeof(GridDev), hipMemcpyHostToDevice));
-        }
+        t.insert(t.end(), st, st + 4);
     }
     return BSN_OK;
 }
 
 static int fmr_refresh(bsn_fmr* m) {
-    std::vector<GridDev> all;
-    for (auto* g : m->lev) all.push_back(g->h);
-    HIPCHK(hipMemcpy(m->d_all, all.data(), all.size() * sizeof(GridDev), hipMemcpyHostToDevice));
+    std::vector<GridDev> t;
+    for (auto* g : m->lev) t.push_back(g->h);
+    if (!m->inplace) CHK(fmr_stage_tables(m, t));
+    CHK(m->all.set(m->ctx, t));
+    m->d_all = m->all.d;
+    m->d_fst = m->all.d + m->nlev;
     for (auto* P : m->plans) CHK(plan_refresh(*P));
-    if (!m->inplace) CHK(fmr_stage_tables(m));
     return BSN_OK;
 }
 
@@ -2157,13 +2333,13 @@ static int fmr_advance(bsn_fmr* m, int l) {
             CHK(fmr_prolong(m, l, 0, true, ProlongDst{3, {g->h.U, g->d_work, g->d_work2}}));
         }
         for (int s = 1; s <= 3; ++s) {
-            const GridDev* T = m->d_fst[4 * l + s - 1];
+            const GridDev* T = m->d_fst + 4 * l + s - 1;
             CHK(plan_fluxes(P, T, 2));
             CHK(stage_update(P, T, s, 0));
             if (child) HIPCHK(launch_fr_coarse(L, P.prec, m->d_all, m->d_f + l, m->hf[l].froff[6] / 5, RK_W[s - 1]));
             if (l > 0) HIPCHK(launch_fr_fine(L, P.prec, m->d_all, m->d_f + (l - 1), m->hf[l - 1].froff[6] / 5, RK_W[s - 1]));
         }
-        CHK(plan_ghost_combine(P, 3, m->d_fst[4 * l + 3]));
+        CHK(plan_ghost_combine(P, 3, m->d_fst + 4 * l + 3));
     } else {
     if (l > 0) HIPCHK(launch_copy_state(L, h, h.U, h.Un));
     if (l > 0) CHK(fmr_interp(m, l));
@@ -2241,6 +2417,7 @@ extern "C" int bsn_fmr_prolong_fine_ghosts(bsn_fmr* m, int level) {
 extern "C" int bsn_fmr_restrict(bsn_fmr* m, int level) {
     if (!m || level < 1 || level >= m->nlev) return set_err(BSN_ERR_ARG, "bad level");
     HIPCHK(hipSetDevice(m->ctx->device));
+    CHK(fmr_refresh(m));
     const FmrDev& f = m->hf[level - 1];
     const int64_t ncells = (int64_t)(f.hi[0] - f.lo[0] + 1) * (f.hi[1] - f.lo[1] + 1) * (f.hi[2] - f.lo[2] + 1);
     HIPCHK(launch_restrict(m->ctx->L(), m->d_all, m->d_f + (level - 1), ncells));
@@ -2343,10 +2520,10 @@ extern "C" int bsn_solve_fmr_poisson(bsn_fmr* m, double* const* phi, int where) 
     std::vector<double*> dst(m->nlev);
     for (int l = 0; l < m->nlev; ++l) dst[l] = where == BSN_HOST ? m->d_sgphi[l] : phi[l];
     CHK(fmr_sg_solve(m, dst.data(), 1.0));
+    HostXfer x(m->ctx);
     if (where == BSN_HOST)
-        for (int l = 0; l < m->nlev; ++l)
-            HIPCHK(hipMemcpyAsync(phi[l], dst[l], active_cells(m->lev[l]->h) * 8, hipMemcpyDeviceToHost,
-                                  m->ctx->stream));
+        for (int l = 0; l < m->nlev; ++l) CHK(x.out(phi[l], dst[l], active_cells(m->lev[l]->h) * 8));
+    CHK(x.flush());
     return sync_ctx(m->ctx);
 }
 
@@ -2371,14 +2548,15 @@ extern "C" int bsn_fmr_prolong_scalar(bsn_fmr* m, int level, const double* phi_c
     // host arrays are staged through the self-gravity buffers of the two levels
     const double* src = phi_c;
     double* dst = where_f == BSN_HOST ? m->d_sgphi[level] : phi_f;
+    HostXfer x(m->ctx);
     if (where_c == BSN_HOST) {
-        HIPCHK(hipMemcpyAsync(m->d_sgphi[level - 1], phi_c, ncn * 8, hipMemcpyHostToDevice, m->ctx->stream));
+        CHK(x.in(m->d_sgphi[level - 1], phi_c, ncn * 8));
         src = m->d_sgphi[level - 1];
     }
     const int nc[3] = {pc.nx, pc.ny, pc.nz}, nf[3] = {cf.nx, cf.ny, cf.nz};
     HIPCHK(launch_prolong_scalar(m->ctx->L(), src, nc, dst, nf, f.lo, f.ratio));
-    if (where_f == BSN_HOST)
-        HIPCHK(hipMemcpyAsync(phi_f, dst, nfn * 8, hipMemcpyDeviceToHost, m->ctx->stream));
+    if (where_f == BSN_HOST) CHK(x.out(phi_f, dst, nfn * 8));
+    CHK(x.flush());
     return sync_ctx(m->ctx);
 }
 
@@ -2411,7 +2589,9 @@ extern "C" int bsn_cfl_dt_fmr3d(bsn_fmr* m, double cfl, double* dt_out) {
     HIPCHK(hipSetDevice(m->ctx->device));
     CHK(fmr_refresh(m));
     CHK(fmr_cfl(m, cfl, 0.0));
-    HIPCHK(hipMemcpyAsync(dt_out, &m->lev[0]->h.scal[SCAL_DT], 8, hipMemcpyDeviceToHost, m->ctx->stream));
+    HostXfer x(m->ctx);
+    CHK(x.out(dt_out, &m->lev[0]->h.scal[SCAL_DT], 8));
+    CHK(x.flush());
     return sync_ctx(m->ctx);
 }
 

@@ -1389,7 +1389,7 @@ __global__ __launch_bounds__(256) void k_cfl(const GridDev* __restrict__ grids,
 
 // dt = cfl / smax (Inf when smax is not > 0), optionally clipped to t_end - t;
 // the maximum is reset for the next accumulation.
-__global__ void k_dt(const GridDev* __restrict__ grids, int ngrids) {
+__global__ void k_dt(const GridDev* __restrict__ grids, int ngrids, double* __restrict__ out) {
     const int g = blockIdx.x * blockDim.x + threadIdx.x;
     if (g >= ngrids) return;
     double* s = grids[g].scal;
@@ -1398,6 +1398,7 @@ __global__ void k_dt(const GridDev* __restrict__ grids, int ngrids) {
     double dt = smax > 0.0 ? s[SCAL_CFL] / smax : __builtin_inf();
     if (s[SCAL_TEND] > 0.0) dt = jl_min(dt, s[SCAL_TEND] - s[SCAL_T]);
     s[SCAL_DT] = dt;
+    if (out) out[g] = dt;
     *(uint64_t*)&s[SCAL_SMAX] = 0;
 }
 
@@ -2347,8 +2348,8 @@ hipError_t launch_floors(const LaunchCtx& L, const GridDev* grids, const int64_t
     return hipGetLastError();
 }
 
-hipError_t launch_dt(const LaunchCtx& L, const GridDev* grids, int ngrids) {
-    hipLaunchKernelGGL(k_dt, dim3((ngrids + 63) / 64), dim3(64), 0, L.stream, grids, ngrids);
+hipError_t launch_dt(const LaunchCtx& L, const GridDev* grids, int ngrids, double* out) {
+    hipLaunchKernelGGL(k_dt, dim3((ngrids + 63) / 64), dim3(64), 0, L.stream, grids, ngrids, out);
     return hipGetLastError();
 }
 

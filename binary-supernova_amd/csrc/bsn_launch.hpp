@@ -47,7 +47,8 @@ hipError_t launch_ghost_combine(const LaunchCtx& L, const GridDev* grids, const 
                                 int ngrids, int64_t total, int stage);
 hipError_t launch_floors(const LaunchCtx& L, const GridDev* grids, const int64_t* off, int ngrids,
                          int64_t total, int copy_un);
-hipError_t launch_dt(const LaunchCtx& L, const GridDev* grids, int ngrids);
+// out: host memory that also takes the ngrids dts, or null
+hipError_t launch_dt(const LaunchCtx& L, const GridDev* grids, int ngrids, double* out = nullptr);
 hipError_t launch_advance_t(const LaunchCtx& L, const GridDev* grids, int ngrids);
 hipError_t launch_set_scal(const LaunchCtx& L, double* scal, int idx, double v);
 hipError_t launch_fill_u64(const LaunchCtx& L, uint64_t* p, int64_t n, uint64_t v);
