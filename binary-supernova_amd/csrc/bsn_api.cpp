@@ -836,19 +836,19 @@ static int plan_floors(Plan& P, int copy_un) {
     return BSN_OK;
 }
 
-static int plan_ghost_combine(Plan& P, int stage, const GridDev* table = nullptr) {
+static int plan_ghost_combine(Plan& P, int stage, const GridDev* table = nullptr, int advance = 0) {
     HIPCHK(launch_ghost_combine(P.ctx->L(), table ? table : P.d_grids, P.d_goff,
-                                (int)P.grids.size(), P.gtotal, stage));
+                                (int)P.grids.size(), P.gtotal, stage, advance));
     return BSN_OK;
 }
 
-static int plan_step_inplace(Plan& P, int fused_cfl);
+static int plan_step_inplace(Plan& P, int device_dt);
 
 // One SSP-RK3 step, out of place (see plan_refresh): per stage the x and y
 // sweeps write their fluxes and one fused kernel computes the z fluxes and
 // finishes every cell.  Bit-identical to the in-place step below.
-static int plan_step(Plan& P, int fused_cfl) {
-    if (P.inplace) return plan_step_inplace(P, fused_cfl);
+static int plan_step(Plan& P, int device_dt) {
+    if (P.inplace) return plan_step_inplace(P, device_dt);
     const LaunchCtx L = P.ctx->L();
     for (int s = 1; s <= 3; ++s) {
         const GridDev* T = P.d_st[s - 1];
@@ -859,15 +859,15 @@ static int plan_step(Plan& P, int fused_cfl) {
             in.U = s == 1 ? g->h.U : s == 2 ? g->h.Un : g->d_work;
             HIPCHK(poisson_solve_state(*g->pois, in, s == 1, g->d_phi, L.stream));
         }
-        CHK(stage_update(P, T, s, fused_cfl && s == 3));
+        CHK(stage_update(P, T, s, device_dt && s == 3));
     }
-    CHK(plan_ghost_combine(P, 3, P.d_st[2]));
+    CHK(plan_ghost_combine(P, 3, P.d_st[2], device_dt));
     return BSN_OK;
 }
 
 // The same step in place with all three flux arrays materialised (the form
 // the FMR levels use, since their flux registers read the z faces).
-static int plan_step_inplace(Plan& P, int fused_cfl) {
+static int plan_step_inplace(Plan& P, int device_dt) {
     for (int s = 1; s <= 3; ++s) {
         if (s == 1) {
             CHK(plan_ghost_fill(P, 1));
@@ -879,19 +879,15 @@ static int plan_step_inplace(Plan& P, int fused_cfl) {
         for (auto* g : P.grids)
             if (g->self_grav)
                 HIPCHK(poisson_solve_state(*g->pois, g->h, 0, g->d_phi, P.ctx->stream));
-        CHK(plan_update(P, s, fused_cfl && s == 3));
+        CHK(plan_update(P, s, device_dt && s == 3));
     }
-    CHK(plan_ghost_combine(P, 3));
+    CHK(plan_ghost_combine(P, 3, nullptr, device_dt));
     return BSN_OK;
 }
 
-static int plan_cfl(Plan& P, double cfl, double t_end) {
+static int plan_cfl(Plan& P, double cfl, double t_end, int restart = 0) {
     const LaunchCtx L = P.ctx->L();
-    for (auto* g : P.grids) {
-        HIPCHK(launch_fill_u64(L, (uint64_t*)&g->h.scal[SCAL_SMAX], 1, 0));
-        HIPCHK(launch_set_scal(L, g->h.scal, SCAL_CFL, cfl));
-        HIPCHK(launch_set_scal(L, g->h.scal, SCAL_TEND, t_end));
-    }
+    HIPCHK(launch_cfl_begin(L, P.d_grids, (int)P.grids.size(), cfl, t_end, restart));
     if (P.small) HIPCHK(launch_cfl(L, 1, P.d_grids, P.d_ut1, P.nut1));
     else         HIPCHK(launch_cfl(L, UPDATE_KZ, P.d_grids, P.d_ut, P.nut));
     return BSN_OK;
@@ -2022,15 +2018,12 @@ extern "C" int bsn_batch_step(bsn_batch* b, const double* dt) {
 static int plan_device_step(Plan& P) {
     const LaunchCtx L = P.ctx->L();
     HIPCHK(launch_dt(L, P.d_grids, (int)P.grids.size()));
-    CHK(plan_step(P, 1));
-    HIPCHK(launch_advance_t(L, P.d_grids, (int)P.grids.size()));
-    return BSN_OK;
+    return plan_step(P, 1);
 }
 
 static int plan_run(Plan& P, double cfl, double t_end, int nsteps, int use_graph) {
     const LaunchCtx L = P.ctx->L();
-    for (auto* g : P.grids) HIPCHK(launch_set_scal(L, g->h.scal, SCAL_T, 0.0));
-    CHK(plan_cfl(P, cfl, t_end));
+    CHK(plan_cfl(P, cfl, t_end, 1));
     bool fft = false;
     for (auto* g : P.grids) fft = fft || g->self_grav;
     if (!use_graph || fft) {     // FFT plans are launched eagerly
@@ -2313,7 +2306,7 @@ static const double RK_W[3] = {1.0 / 6.0, 1.0 / 6.0, 2.0 / 3.0};   // fmr3d.jl:4
 
 // Advance level l by its dt (already in its scal): own RK3 with flux-register
 // accumulation, then the child's sub-cycles, restriction and correction.
-static int fmr_advance(bsn_fmr* m, int l) {
+static int fmr_advance(bsn_fmr* m, int l, int device_dt = 0) {
     Plan& P = *m->plans[l];
     const LaunchCtx L = m->ctx->L();
     const bool child = l + 1 < m->nlev;
@@ -2339,7 +2332,7 @@ static int fmr_advance(bsn_fmr* m, int l) {
             if (child) HIPCHK(launch_fr_coarse(L, P.prec, m->d_all, m->d_f + l, m->hf[l].froff[6] / 5, RK_W[s - 1]));
             if (l > 0) HIPCHK(launch_fr_fine(L, P.prec, m->d_all, m->d_f + (l - 1), m->hf[l - 1].froff[6] / 5, RK_W[s - 1]));
         }
-        CHK(plan_ghost_combine(P, 3, m->d_fst + 4 * l + 3));
+        CHK(plan_ghost_combine(P, 3, m->d_fst + 4 * l + 3, device_dt));
     } else {
     if (l > 0) HIPCHK(launch_copy_state(L, h, h.U, h.Un));
     if (l > 0) CHK(fmr_interp(m, l));
@@ -2356,19 +2349,15 @@ static int fmr_advance(bsn_fmr* m, int l) {
         if (l > 0) HIPCHK(launch_fr_fine(L, P.prec, m->d_all, m->d_f + (l - 1), m->hf[l - 1].froff[6] / 5, RK_W[s - 1]));
         CHK(plan_update(P, s, 0));
     }
-    CHK(plan_ghost_combine(P, 3));
+    CHK(plan_ghost_combine(P, 3, nullptr, device_dt));
     }
     if (child) {
         const FmrDev& f = m->hf[l];
-        HIPCHK(launch_child_dt(L, m->d_all, l, l + 1, f.ratio));
         for (int ss = 0; ss < f.ratio; ++ss) {
             m->alpha[l + 1] = (double)ss / (double)f.ratio;
             CHK(fmr_advance(m, l + 1));
         }
-        const int64_t ncells = (int64_t)(f.hi[0] - f.lo[0] + 1) * (f.hi[1] - f.lo[1] + 1) * (f.hi[2] - f.lo[2] + 1);
-        HIPCHK(launch_restrict(L, m->d_all, m->d_f + l, ncells));
-        HIPCHK(launch_bc_correct(L, m->d_all, m->d_f + l, f.froff[6] / 5));
-        HIPCHK(launch_floors_box(L, m->d_all, m->d_f + l, f));
+        HIPCHK(launch_fmr_correct(L, m->d_all, m->d_f + l, f));
     }
     return BSN_OK;
 }
@@ -2570,17 +2559,14 @@ extern "C" int bsn_fmr_set_self_gravity(bsn_fmr* m, int on, double G_grav) {
 
 // Level CFL dts folded into the root: dt_0 = min(dt_0, r0 dt_1, r0 r1 dt_2, ...)
 static int fmr_cfl(bsn_fmr* m, double cfl, double t_end) {
-    const LaunchCtx L = m->ctx->L();
-    double factor = 1.0;
+    FmrFactors f{};
+    f.nlev = m->nlev;
+    f.factor[0] = 1.0;
     for (int l = 0; l < m->nlev; ++l) {
-        Plan& P = *m->plans[l];
-        CHK(plan_cfl(P, cfl, l == 0 ? t_end : 0.0));
-        HIPCHK(launch_dt(L, P.d_grids, 1));
+        if (l > 0) f.factor[l] = f.factor[l - 1] * (double)m->hf[l - 1].ratio;
+        CHK(plan_cfl(*m->plans[l], cfl, l == 0 ? t_end : 0.0));
     }
-    for (int l = 1; l < m->nlev; ++l) {
-        factor *= (double)m->hf[l - 1].ratio;
-        HIPCHK(launch_fold_dt(L, m->d_all, 0, l, factor));
-    }
+    HIPCHK(launch_fmr_dt(m->ctx->L(), m->d_all, f));
     return BSN_OK;
 }
 
@@ -2600,9 +2586,7 @@ extern "C" int bsn_cfl_dt_fmr3d(bsn_fmr* m, double cfl, double* dt_out) {
 static int fmr_device_step(bsn_fmr* m, double cfl, double t_end) {
     CHK(fmr_cfl(m, cfl, t_end));
     if (m->sg_on) CHK(fmr_sg_solve(m, m->d_sgphi.data(), m->sg_G));
-    CHK(fmr_advance(m, 0));
-    HIPCHK(launch_advance_t(m->ctx->L(), m->d_all, 1));
-    return BSN_OK;
+    return fmr_advance(m, 0, 1);
 }
 
 extern "C" int bsn_fmr_run(bsn_fmr* m, double cfl, double t_end, int nsteps, int use_graph) {

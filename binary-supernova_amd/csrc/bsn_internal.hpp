@@ -138,6 +138,12 @@ BSN_HD static inline ProlongWork prolong_work(int nx, int ny, int nz, int all_ce
 #define ZT_LEN_SHIFT 21
 #define ZT_MAX_LEN 1023
 
+// Per level of a hierarchy, its steps per root step.
+struct FmrFactors {
+    int nlev;
+    double factor[BSN_MAXLEV];
+};
+
 // FMR coupling between a parent grid and the nested child grid.
 struct FmrDev {
     int parent, child;        // grid indices into the GridDev table

@@ -14,7 +14,7 @@
 //   _prolong_fine_ghosts!/_prolong_all!  fmr3d.jl:206-255     k_prolong
 //   _restrict!                        fmr3d.jl:266-285        k_restrict
 //   _accumulate_fr_coarse!/_fine!     fmr3d.jl:292-369        k_fr_coarse, k_fr_fine
-//   _bc_correct!                      fmr3d.jl:379-422        k_bc_correct
+//   _bc_correct!                      fmr3d.jl:379-422        k_fmr_correct (with _restrict! and floors)
 //
 // All work is described by device-resident tile lists (struct Tile) or by
 // per-grid prefix offsets, so one launch sweeps any number of grids of any
@@ -175,8 +175,14 @@ __global__ void k_ghost_fill(const GridDev* __restrict__ grids, const int64_t* _
 // (euler3d.jl:138 fills dU with zeros; the combine runs over the whole array).
 // With ghost mapping the stage input's ghost value is read from the active
 // cell it maps to.
+// advance: the step ends here, t += dt.
 __global__ void k_ghost_combine(const GridDev* __restrict__ grids, const int64_t* __restrict__ off,
-                                int ngrids, int stage) {
+                                int ngrids, int stage, int advance) {
+    if (advance && blockIdx.x == 0)
+        for (int g = threadIdx.x; g < ngrids; g += blockDim.x) {
+            double* s = grids[g].scal;
+            s[SCAL_T] = s[SCAL_T] + s[SCAL_DT];
+        }
     const int64_t total = off[ngrids];
     for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < total;
          e += (int64_t)gridDim.x * blockDim.x) {
@@ -1389,24 +1395,43 @@ __global__ __launch_bounds__(256) void k_cfl(const GridDev* __restrict__ grids,
 
 // dt = cfl / smax (Inf when smax is not > 0), optionally clipped to t_end - t;
 // the maximum is reset for the next accumulation.
-__global__ void k_dt(const GridDev* __restrict__ grids, int ngrids, double* __restrict__ out) {
-    const int g = blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= ngrids) return;
-    double* s = grids[g].scal;
+__device__ __forceinline__ double take_dt(double* s) {
     const uint64_t bits = *(const uint64_t*)&s[SCAL_SMAX];
     const double smax = __longlong_as_double((long long)bits);
     double dt = smax > 0.0 ? s[SCAL_CFL] / smax : __builtin_inf();
     if (s[SCAL_TEND] > 0.0) dt = jl_min(dt, s[SCAL_TEND] - s[SCAL_T]);
     s[SCAL_DT] = dt;
-    if (out) out[g] = dt;
     *(uint64_t*)&s[SCAL_SMAX] = 0;
+    return dt;
 }
 
-__global__ void k_advance_t(const GridDev* __restrict__ grids, int ngrids) {
+__global__ void k_dt(const GridDev* __restrict__ grids, int ngrids, double* __restrict__ out) {
+    const int g = blockIdx.x * blockDim.x + threadIdx.x;
+    if (g >= ngrids) return;
+    const double dt = take_dt(grids[g].scal);
+    if (out) out[g] = dt;
+}
+
+// The dts of a hierarchy's levels, then dt_root = min(dt_root, r0 dt_1, r0 r1 dt_2, ...)
+// (cfl_dt_fmr3d, fmr3d.jl:615-622; factor[l] the ratios' product up to level l).
+__global__ void k_fmr_dt(const GridDev* __restrict__ grids, FmrFactors f) {
+    double* root = grids[0].scal;
+    double dt = take_dt(root);
+    for (int l = 1; l < f.nlev; ++l) dt = jl_min(dt, take_dt(grids[l].scal) * f.factor[l]);
+    root[SCAL_DT] = dt;
+}
+
+// Start of a CFL accumulation: CFL number, end time and an empty maximum; restart
+// also sets t = 0.  One launch for all grids: three per grid were 0.6 of the 14 ms of
+// two steps of 48 problems.
+__global__ void k_cfl_begin(const GridDev* __restrict__ grids, int ngrids, double cfl, double t_end, int restart) {
     const int g = blockIdx.x * blockDim.x + threadIdx.x;
     if (g >= ngrids) return;
     double* s = grids[g].scal;
-    s[SCAL_T] = s[SCAL_T] + s[SCAL_DT];
+    s[SCAL_CFL] = cfl;
+    s[SCAL_TEND] = t_end;
+    *(uint64_t*)&s[SCAL_SMAX] = 0;
+    if (restart) s[SCAL_T] = 0.0;
 }
 
 __global__ void k_set_scal(double* scal, int idx, double v) { scal[idx] = v; }
@@ -1828,12 +1853,15 @@ __global__ void k_time_interp(const GridDev* __restrict__ grids, const FmrDev* _
 // Start of a level's fused step: its ghost cells, which the stage-3 combination
 // reads after the prolongation has replaced them, are saved to Un (a child, own
 // != 0); so is what its child's ghost stencils read of the state at the start,
-// and the child's flux registers are cleared (a parent, fmr != null).  Copying
+// the child's flux registers are cleared and its dt is set (a parent, fmr != null).  Copying
 // the whole state took 258 of 6270 us per root step of three levels from 192^3,
 // now 90.
 __global__ void k_level_begin(const GridDev* __restrict__ grids, int level, const FmrDev* __restrict__ fmr,
                               int own) {
     const GridDev& G = grids[level];
+    // dt_child = dt_parent / ratio (fmr3d.jl:454)
+    if (fmr && blockIdx.x == 0 && threadIdx.x == 0)
+        grids[fmr->child].scal[SCAL_DT] = G.scal[SCAL_DT] / (double)fmr->ratio;
     int64_t nb = 0, nr = 0;
     int nx = 1, ny = 1;
     if (fmr) {
@@ -1864,23 +1892,6 @@ __global__ void k_level_begin(const GridDev* __restrict__ grids, int level, cons
         const int64_t c = uidx(G, i, j, k);
 #pragma unroll
         for (int q = 0; q < 5; ++q) G.Un[q * G.fs + c] = G.U[q * G.fs + c];
-    }
-}
-
-// Floors on the cells of a parent that restriction and flux correction changed:
-// the child's box and one cell around it.  The others were floored by the last
-// stage, and a floored cell stays as it is under the floors.
-__global__ void k_floors_box(const GridDev* __restrict__ grids, const FmrDev* __restrict__ fmr) {
-    const FmrDev& M = *fmr;
-    const GridDev& G = grids[M.parent];
-    const int i0 = max(M.lo[0] - 1, 1), j0 = max(M.lo[1] - 1, 1), k0 = max(M.lo[2] - 1, 1);
-    const int nx = min(M.hi[0] + 1, G.nx) - i0 + 1, ny = min(M.hi[1] + 1, G.ny) - j0 + 1;
-    const int64_t total = (int64_t)nx * ny * (min(M.hi[2] + 1, G.nz) - k0 + 1);
-    for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < total;
-         e += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t r = e / nx;
-        floor_cell(G, uidx(G, NG - 1 + i0 + (int)(e % nx), NG - 1 + j0 + (int)(r % ny), NG - 1 + k0 + (int)(r / ny)),
-                   false);
     }
 }
 
@@ -2043,47 +2054,64 @@ __global__ void k_fr_fine(const GridDev* __restrict__ grids, const FmrDev* __res
     }
 }
 
-// _bc_correct! (fmr3d.jl:379-422): every corrected coarse cell receives one
-// face's correction, so the faces are applied in parallel.
-__global__ void k_bc_correct(const GridDev* __restrict__ grids, const FmrDev* __restrict__ fmr) {
+// _restrict! (fmr3d.jl:266-285) into the child's box, _bc_correct! (fmr3d.jl:379-422)
+// on the cells around it, each of which receives one face's correction, and the
+// floors on both: the parent's other cells were floored by the last stage, and a
+// floored cell stays as it is under the floors.
+__global__ void k_fmr_correct(const GridDev* __restrict__ grids, const FmrDev* __restrict__ fmr) {
     const FmrDev& M = *fmr;
     const GridDev& C = grids[M.parent];
-    const int64_t n = M.froff[6] / 5;
-    for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < n;
+    const GridDev& Fg = grids[M.child];
+    const int r = M.ratio;
+    int n[3];
+    for (int a = 0; a < 3; ++a) n[a] = M.hi[a] - M.lo[a] + 1;
+    const int64_t total = (int64_t)(n[0] + 2) * (n[1] + 2) * (n[2] + 2);
+    const double inv_r3 = 1.0 / (double)(r * r * r);
+    for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < total;
          e += (int64_t)gridDim.x * blockDim.x) {
-        int face = 0;
-        while (face < 5 && e >= M.froff[face + 1] / 5) ++face;
-        const int64_t loc = e - M.froff[face] / 5;
-        int n1, n2;
-        face_dims(M, face, n1, n2);
-        const int a = (int)(loc % n1), b = (int)(loc / n1);
-        const int hi = face & 1;
-        int ci, cj, ck;   // 1-based coarse active
-        double inv;
-        if (face < 2)      { ci = hi ? M.hi[0] + 1 : M.lo[0] - 1; cj = M.lo[1] + a; ck = M.lo[2] + b; inv = C.idx; }
-        else if (face < 4) { ci = M.lo[0] + a; cj = hi ? M.hi[1] + 1 : M.lo[1] - 1; ck = M.lo[2] + b; inv = C.idy; }
-        else               { ci = M.lo[0] + a; cj = M.lo[1] + b; ck = hi ? M.hi[2] + 1 : M.lo[2] - 1; inv = C.idz; }
-        const int64_t c = uidx(C, NG + ci - 1, NG + cj - 1, NG + ck - 1);
-        for (int q = 0; q < 5; ++q) {
-            const double rc = M.frc[M.froff[face] + q + 5 * loc];
-            const double rf = M.frf[M.froff[face] + q + 5 * loc];
-            const double delta = hi ? (rf - rc) * inv : (rc - rf) * inv;
-            C.U[q * C.fs + c] += delta;
+        // position in the box, -1 and n outside it
+        const int64_t t = e / (n[0] + 2);
+        const int m[3] = {(int)(e % (n[0] + 2)) - 1, (int)(t % (n[1] + 2)) - 1, (int)(t / (n[1] + 2)) - 1};
+        int face = -1, outside = 0;
+#pragma unroll
+        for (int a = 0; a < 3; ++a)
+            if (m[a] < 0 || m[a] == n[a]) { ++outside; face = 2 * a + (m[a] < 0 ? 0 : 1); }
+        if (outside > 1) continue;
+        const int i = M.lo[0] - 1 + m[0], j = M.lo[1] - 1 + m[1], k = M.lo[2] - 1 + m[2];   // 0-based active
+        const int64_t c = uidx(C, NG + i, NG + j, NG + k);
+        double u[5];
+        if (outside == 0) {
+#pragma unroll
+            for (int q = 0; q < 5; ++q) u[q] = 0.0;
+            for (int sx = 0; sx < r; ++sx)
+                for (int sy = 0; sy < r; ++sy)
+                    for (int sz = 0; sz < r; ++sz) {
+                        const int64_t o = uidx(Fg, NG + r * m[0] + sx, NG + r * m[1] + sy, NG + r * m[2] + sz);
+#pragma unroll
+                        for (int q = 0; q < 5; ++q) u[q] += Fg.U[q * Fg.fs + o];
+                    }
+#pragma unroll
+            for (int q = 0; q < 5; ++q) u[q] = u[q] * inv_r3;
+        } else {
+            const int n1 = face < 2 ? n[1] : n[0];
+            const int a = face < 2 ? m[1] : m[0], b = face < 4 ? m[2] : m[1];
+            const double inv = face < 2 ? C.idx : face < 4 ? C.idy : C.idz;
+            const int64_t o = M.froff[face] + 5 * ((int64_t)b * n1 + a);
+#pragma unroll
+            for (int q = 0; q < 5; ++q) {
+                const double rc = M.frc[o + q], rf = M.frf[o + q];
+                u[q] = C.U[q * C.fs + c] + ((face & 1) ? (rf - rc) * inv : (rc - rf) * inv);
+            }
         }
+        if (i >= 0 && i < C.nx && j >= 0 && j < C.ny && k >= 0 && k < C.nz) {
+            if (C.prec == 1) apply_floor<true>(u, C.rho_floor, C.P_floor, C.gamma);
+            else             apply_floor<false>(u, C.rho_floor, C.P_floor, C.gamma);
+        }
+#pragma unroll
+        for (int q = 0; q < 5; ++q) C.U[q * C.fs + c] = u[q];
     }
 }
 
-// dt of a nested level: dt_child = dt_parent / ratio (fmr3d.jl:454).
-__global__ void k_child_dt(const GridDev* __restrict__ grids, int parent, int child, int ratio) {
-    grids[child].scal[SCAL_DT] = grids[parent].scal[SCAL_DT] / (double)ratio;
-}
-
-// dt_c = min(dt_c, r * dt_f) over a hierarchy (cfl_dt_fmr3d, fmr3d.jl:616-622):
-// level dts are computed first by k_dt on every grid, then folded into the root.
-__global__ void k_fold_dt(const GridDev* __restrict__ grids, int root, int child, double factor) {
-    double* s = grids[root].scal;
-    s[SCAL_DT] = jl_min(s[SCAL_DT], factor * grids[child].scal[SCAL_DT]);
-}
 
 // ---------------------------------------------------------------------------
 // Launch helpers
@@ -2333,10 +2361,10 @@ hipError_t launch_ghost_fill(const LaunchCtx& L, const GridDev* grids, const int
 }
 
 hipError_t launch_ghost_combine(const LaunchCtx& L, const GridDev* grids, const int64_t* off,
-                                int ngrids, int64_t total, int stage) {
+                                int ngrids, int64_t total, int stage, int advance) {
     if (total <= 0) return hipSuccess;
     hipLaunchKernelGGL(k_ghost_combine, dim3(flat_blocks(total, L.cus)), dim3(256), 0, L.stream,
-                       grids, off, ngrids, stage);
+                       grids, off, ngrids, stage, advance);
     return hipGetLastError();
 }
 
@@ -2348,13 +2376,27 @@ hipError_t launch_floors(const LaunchCtx& L, const GridDev* grids, const int64_t
     return hipGetLastError();
 }
 
-hipError_t launch_dt(const LaunchCtx& L, const GridDev* grids, int ngrids, double* out) {
-    hipLaunchKernelGGL(k_dt, dim3((ngrids + 63) / 64), dim3(64), 0, L.stream, grids, ngrids, out);
+hipError_t launch_fmr_dt(const LaunchCtx& L, const GridDev* grids, const FmrFactors& f) {
+    hipLaunchKernelGGL(k_fmr_dt, dim3(1), dim3(1), 0, L.stream, grids, f);
     return hipGetLastError();
 }
 
-hipError_t launch_advance_t(const LaunchCtx& L, const GridDev* grids, int ngrids) {
-    hipLaunchKernelGGL(k_advance_t, dim3((ngrids + 63) / 64), dim3(64), 0, L.stream, grids, ngrids);
+hipError_t launch_cfl_begin(const LaunchCtx& L, const GridDev* grids, int ngrids, double cfl, double t_end,
+                            int restart) {
+    hipLaunchKernelGGL(k_cfl_begin, dim3((ngrids + 63) / 64), dim3(64), 0, L.stream, grids, ngrids, cfl, t_end,
+                       restart);
+    return hipGetLastError();
+}
+
+hipError_t launch_fmr_correct(const LaunchCtx& L, const GridDev* grids, const FmrDev* fmr, const FmrDev& hf) {
+    int64_t cells = 1;
+    for (int a = 0; a < 3; ++a) cells *= hf.hi[a] - hf.lo[a] + 3;
+    hipLaunchKernelGGL(k_fmr_correct, dim3(flat_blocks(cells, L.cus)), dim3(256), 0, L.stream, grids, fmr);
+    return hipGetLastError();
+}
+
+hipError_t launch_dt(const LaunchCtx& L, const GridDev* grids, int ngrids, double* out) {
+    hipLaunchKernelGGL(k_dt, dim3((ngrids + 63) / 64), dim3(64), 0, L.stream, grids, ngrids, out);
     return hipGetLastError();
 }
 
@@ -2499,13 +2541,6 @@ hipError_t launch_level_begin(const LaunchCtx& L, const GridDev* grids, int leve
     return hipGetLastError();
 }
 
-hipError_t launch_floors_box(const LaunchCtx& L, const GridDev* grids, const FmrDev* fmr, const FmrDev& hf) {
-    int64_t box = 1;
-    for (int a = 0; a < 3; ++a) box *= hf.hi[a] - hf.lo[a] + 3;
-    hipLaunchKernelGGL(k_floors_box, dim3(flat_blocks(box, L.cus)), dim3(256), 0, L.stream, grids, fmr);
-    return hipGetLastError();
-}
-
 hipError_t launch_fr_coarse(const LaunchCtx& L, int prec, const GridDev* grids, const FmrDev* fmr,
                             int64_t nelem, double weight) {
     const dim3 grid(flat_blocks(nelem, L.cus), 5);     // one grid row per field
@@ -2523,21 +2558,6 @@ hipError_t launch_fr_fine(const LaunchCtx& L, int prec, const GridDev* grids, co
         hipLaunchKernelGGL(k_fr_fine<double>, grid, dim3(256), 0, L.stream, grids, fmr, weight);
     else
         hipLaunchKernelGGL(k_fr_fine<float>, grid, dim3(256), 0, L.stream, grids, fmr, weight);
-    return hipGetLastError();
-}
-
-hipError_t launch_bc_correct(const LaunchCtx& L, const GridDev* grids, const FmrDev* fmr, int64_t nelem) {
-    hipLaunchKernelGGL(k_bc_correct, dim3(flat_blocks(nelem, L.cus)), dim3(256), 0, L.stream, grids, fmr);
-    return hipGetLastError();
-}
-
-hipError_t launch_child_dt(const LaunchCtx& L, const GridDev* grids, int parent, int child, int ratio) {
-    hipLaunchKernelGGL(k_child_dt, dim3(1), dim3(1), 0, L.stream, grids, parent, child, ratio);
-    return hipGetLastError();
-}
-
-hipError_t launch_fold_dt(const LaunchCtx& L, const GridDev* grids, int root, int child, double factor) {
-    hipLaunchKernelGGL(k_fold_dt, dim3(1), dim3(1), 0, L.stream, grids, root, child, factor);
     return hipGetLastError();
 }
 

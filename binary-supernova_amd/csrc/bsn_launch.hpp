@@ -44,12 +44,15 @@ hipError_t launch_zupdate(const LaunchCtx& L, int prec, int shape, const GridDev
 hipError_t launch_ghost_fill(const LaunchCtx& L, const GridDev* grids, const int64_t* off,
                              int ngrids, int64_t total, int copy_un);
 hipError_t launch_ghost_combine(const LaunchCtx& L, const GridDev* grids, const int64_t* off,
-                                int ngrids, int64_t total, int stage);
+                                int ngrids, int64_t total, int stage, int advance);
 hipError_t launch_floors(const LaunchCtx& L, const GridDev* grids, const int64_t* off, int ngrids,
                          int64_t total, int copy_un);
+hipError_t launch_cfl_begin(const LaunchCtx& L, const GridDev* grids, int ngrids, double cfl, double t_end,
+                            int restart);
+hipError_t launch_fmr_dt(const LaunchCtx& L, const GridDev* grids, const FmrFactors& f);
+hipError_t launch_fmr_correct(const LaunchCtx& L, const GridDev* grids, const FmrDev* fmr, const FmrDev& hf);
 // out: host memory that also takes the ngrids dts, or null
 hipError_t launch_dt(const LaunchCtx& L, const GridDev* grids, int ngrids, double* out = nullptr);
-hipError_t launch_advance_t(const LaunchCtx& L, const GridDev* grids, int ngrids);
 hipError_t launch_set_scal(const LaunchCtx& L, double* scal, int idx, double v);
 hipError_t launch_fill_u64(const LaunchCtx& L, uint64_t* p, int64_t n, uint64_t v);
 hipError_t launch_aos_to_soa(const LaunchCtx& L, const GridDev& G, const double* aos, double* dst);
@@ -91,13 +94,9 @@ hipError_t launch_prolong_scalar(const LaunchCtx& L, const double* phc, const in
 hipError_t launch_scale(const LaunchCtx& L, double* a, int64_t n, double s);
 hipError_t launch_level_begin(const LaunchCtx& L, const GridDev* grids, int level, const GridDev& h,
                               const FmrDev* fmr, const FmrDev* hf, int own);
-hipError_t launch_floors_box(const LaunchCtx& L, const GridDev* grids, const FmrDev* fmr, const FmrDev& hf);
 hipError_t launch_fr_coarse(const LaunchCtx& L, int prec, const GridDev* grids, const FmrDev* fmr,
                             int64_t nelem, double weight);
 hipError_t launch_fr_fine(const LaunchCtx& L, int prec, const GridDev* grids, const FmrDev* fmr,
                           int64_t nelem, double weight);
-hipError_t launch_bc_correct(const LaunchCtx& L, const GridDev* grids, const FmrDev* fmr, int64_t nelem);
-hipError_t launch_child_dt(const LaunchCtx& L, const GridDev* grids, int parent, int child, int ratio);
-hipError_t launch_fold_dt(const LaunchCtx& L, const GridDev* grids, int root, int child, double factor);
 
 }  // namespace bsn
