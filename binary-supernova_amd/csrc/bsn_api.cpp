@@ -92,13 +92,16 @@ struct bsn_ctx {
 // on numpy arrays takes 0.19 ms per step at 8^3 (0.50 by the runtime's copies), 0.60
 // at 32^3 (0.82), 2.1 at 64^3 (2.5).  Three helper threads doubled the copying, but
 // their start cost a 4 MB array more (40^3 1.43 ms against 0.93) than they gave a
-// 14 MB one.  Memory that is pinned already is copied directly.
+// 14 MB one.  Memory that is pinned already (or managed) is copied directly, and
+// the copy waited for: the caller may write to it, or free it, as soon as it has
+// it back.
 //
 // The object holds the pipe for as long as it lives; data has arrived in host
 // arrays after flush().
 class HostXfer {
     bsn_ctx* c;
     std::lock_guard<std::mutex> lk;
+    bool direct = false;     // a copy straight to the caller's memory is in flight
     struct Out { char* dst; size_t n; int slot; } q[HostPipe::SLOTS];    // not taken yet, oldest first
     int qn = 0;
 
@@ -154,16 +157,19 @@ class HostXfer {
 public:
     explicit HostXfer(bsn_ctx* ctx) : c(ctx), lk(ctx->pipe.mu) {}
     ~HostXfer() {
-        // after an error: nothing may still be on its way to a slot
-        if (qn > 0) (void)hipStreamSynchronize(c->stream);
+        // after an error: nothing may still be on its way to a slot or an array
+        if (qn > 0 || direct) (void)hipStreamSynchronize(c->stream);
     }
     HostXfer(const HostXfer&) = delete;
     HostXfer& operator=(const HostXfer&) = delete;
 
     // on return src has been read
     int in(void* dst, const void* src, size_t n) {
-        if (n > DIRECT_FROM || !pageable(src)) {
+        const bool paged = pageable(src);
+        if (n > DIRECT_FROM || !paged) {
+            // from pageable memory the runtime's copy returns when it has read it
             HIPCHK(hipMemcpyAsync(dst, src, n, hipMemcpyHostToDevice, c->stream));
+            if (!paged) HIPCHK(hipStreamSynchronize(c->stream));
             return BSN_OK;
         }
         CHK(ready());
@@ -180,6 +186,7 @@ public:
     int out(void* dst, const void* src, size_t n) {
         if (!pageable(dst)) {
             HIPCHK(hipMemcpyAsync(dst, src, n, hipMemcpyDeviceToHost, c->stream));
+            direct = true;
             return BSN_OK;
         }
         CHK(ready());
@@ -195,6 +202,8 @@ public:
     }
     int flush() {
         while (qn > 0) CHK(take());
+        if (direct) HIPCHK(hipStreamSynchronize(c->stream));
+        direct = false;
         return BSN_OK;
     }
     // host memory that a kernel can write; read it after the stream is done
