@@ -1331,7 +1331,11 @@ extern "C" int bsn_grid_set_phi(bsn_grid* g, const double* phi, int where) {
         HostXfer x(g->ctx);
         CHK(x.in(g->d_phi, phi, bytes));
     } else {
+        // after what the null stream still has to write to phi; such a copy may be
+        // on its way when hipMemcpy returns, and neither the caller's next write
+        // nor the context's stream would wait for it
         HIPCHK(hipMemcpy(g->d_phi, phi, bytes, hipMemcpyDeviceToDevice));
+        HIPCHK(hipStreamSynchronize(nullptr));
     }
     g->h.phi = g->d_phi;
     return grid_changed(g);

@@ -1,0 +1,96 @@
+"""GPU: the library's stream against the null stream, on which callers prepare
+device memory (torch's default stream is it): the null stream is given some
+milliseconds of copies first, so that an ordering that is missing shows."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import binary_supernova_amd as bsn
+from binary_supernova_amd import problems as P
+from binary_supernova_amd._lib import BSN_DEVICE, call
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+D = (0.1, 0.07, 0.13)
+D2D, H2D = 3, 1
+
+
+class Hip:
+    """The HIP runtime that libbsn_hip.so itself links."""
+
+    def __init__(self):
+        bsn.load()
+        L = self.L = C.CDLL("/opt/rocm/lib/libamdhip64.so")
+        p, n = C.c_void_p, C.c_size_t
+        L.hipMalloc.argtypes, L.hipFree.argtypes = [C.POINTER(p), n], [p]
+        L.hipMemcpy.argtypes, L.hipMemcpyAsync.argtypes = [p, p, n, C.c_int], [p, p, n, C.c_int, p]
+        L.hipStreamCreateWithFlags.argtypes = [C.POINTER(p), C.c_uint]
+        L.hipStreamDestroy.argtypes = L.hipStreamSynchronize.argtypes = [p]
+        self.held = []
+
+    def __getattr__(self, name):
+        def run(*a):
+            assert getattr(self.L, name)(*a) == 0, name
+        return run
+
+    def buffer(self, n, values=None):
+        p = C.c_void_p()
+        self.hipMalloc(C.byref(p), n)
+        self.held.append(p)
+        if values is not None:
+            self.hipMemcpy(p, values.ctypes.data, values.nbytes, H2D)
+        return p
+
+    def keep_null_stream_busy(self):
+        n = 512 << 20
+        a, b = self.buffer(n), self.buffer(n)
+        for _ in range(60):
+            self.hipMemcpyAsync(a, b, n, D2D, None)
+
+    def close(self):
+        self.L.hipDeviceSynchronize()
+        for p in self.held:
+            self.L.hipFree(p)
+
+
+@pytest.fixture
+def hip():
+    h = Hip()
+    yield h
+    h.close()
+
+
+def state(shape, seed):
+    rng = np.random.default_rng(seed)
+    U = P.empty_state(*shape)
+    s = U.shape[:-1]
+    rho, p = rng.uniform(0.5, 2.0, s), rng.uniform(0.5, 2.0, s)
+    v = rng.normal(0.0, 0.3, s + (3,))
+    U[..., 0], U[..., 1:4] = rho, rho[..., None] * v
+    U[..., 4] = p / 0.4 + 0.5 * rho * (v * v).sum(-1)
+    return U
+
+
+def test_phi_from_device_memory(hip):
+    # phi reaches the caller's buffer late, in the null stream's order, and the
+    # buffer is written again on a stream of its own once the call is back
+    print("device phi", flush=True)
+    shape = (24, 18, 20)
+    U, phi = state(shape, 1), 0.1 * np.random.default_rng(2).normal(size=shape[::-1])
+    src, buf = hip.buffer(phi.nbytes, phi), hip.buffer(phi.nbytes, np.full_like(phi, 5.0))
+    other = hip.buffer(phi.nbytes, np.full_like(phi, 7.0))
+    g = bsn.Grid(*shape).set_state(U)
+    g.set_params(*D, 1.4)
+    s = C.c_void_p()
+    hip.hipStreamCreateWithFlags(C.byref(s), 1)
+    hip.keep_null_stream_busy()
+    hip.hipMemcpyAsync(buf, src, phi.nbytes, D2D, None)
+    call("bsn_grid_set_phi", g.handle, buf, BSN_DEVICE)
+    hip.hipMemcpyAsync(buf, other, phi.nbytes, D2D, s)
+    bsn.euler3d_step_(g, *shape, *D, 2e-3, 1.4)
+    O.euler3d_step(U, *D, 2e-3, 1.4, "outflow", phi=phi)
+    np.testing.assert_array_equal(g.get_state(), U)
+    hip.hipStreamSynchronize(s)
+    hip.hipStreamDestroy(s)
