@@ -635,19 +635,18 @@ static int plan_set_shape(Plan& P, int dir, int shape) {
     return BSN_OK;
 }
 
-static int ensure_work(bsn_grid* g) {
-    if (g->d_work) return BSN_OK;
-    HIPCHK(hipMalloc((void**)&g->d_work, 5 * g->h.fs * 8));
-    HIPCHK(hipMemset(g->d_work, 0, 5 * g->h.fs * 8));
+// A work buffer in U's layout, cleared (its padding stays so) on the context's
+// stream, ahead of the kernels that write it: a hipMemset on the null stream
+// could run after them.
+static int ensure_buffer(bsn_grid* g, double*& d) {
+    if (d) return BSN_OK;
+    HIPCHK(hipMalloc((void**)&d, 5 * g->h.fs * 8));
+    HIPCHK(launch_fill_u64(g->ctx->L(), (uint64_t*)d, 5 * g->h.fs, 0));
     return BSN_OK;
 }
-
-static int ensure_work2(bsn_grid* g) {
-    if (g->d_work2) return BSN_OK;
-    HIPCHK(hipMalloc((void**)&g->d_work2, 5 * g->h.fs * 8));
-    HIPCHK(hipMemset(g->d_work2, 0, 5 * g->h.fs * 8));
-    return BSN_OK;
-}
+static int ensure_work(bsn_grid* g) { return ensure_buffer(g, g->d_work); }
+static int ensure_work2(bsn_grid* g) { return ensure_buffer(g, g->d_work2); }
+static int ensure_scratch(bsn_grid* g) { return ensure_buffer(g, g->d_scratch); }
 
 // Descriptor tables.  In-place table: U = Uout = the state, Un = base copy.
 // Out-of-place step with the state A, B = the Un buffer and C = the work
@@ -1058,13 +1057,6 @@ static int ensure_stage(bsn_grid* g, size_t bytes) {
     g->stage_bytes = 0;
     HIPCHK(hipMalloc((void**)&g->d_stage, bytes));
     g->stage_bytes = bytes;
-    return BSN_OK;
-}
-
-static int ensure_scratch(bsn_grid* g) {
-    if (g->d_scratch) return BSN_OK;
-    HIPCHK(hipMalloc((void**)&g->d_scratch, 5 * g->h.fs * 8));
-    HIPCHK(hipMemset(g->d_scratch, 0, 5 * g->h.fs * 8));
     return BSN_OK;
 }
 

@@ -94,3 +94,25 @@ def test_phi_from_device_memory(hip):
     np.testing.assert_array_equal(g.get_state(), U)
     hip.hipStreamSynchronize(s)
     hip.hipStreamDestroy(s)
+
+
+def test_work_buffers_made_beside_a_busy_null_stream(hip):
+    # the right-hand side's scratch and the levels' second work buffer are made,
+    # and cleared, by the first call that needs them
+    print("work buffers", flush=True)
+    d, n, box, r = 0.1, (20, 18, 16), (6, 13, 5, 12, 5, 10), 2
+    nf = tuple((box[2 * a + 1] - box[2 * a] + 1) * r for a in range(3))
+    U, Uf = state(n, 3), state(nf, 4)
+    g = bsn.Grid(*n).set_state(U)
+    bsn.cfl_dt_3d(g, *n, d, d, d, 1.4, 0.3)
+    H = bsn.FMRHierarchy([n, nf], [(d,) * 3, (d / r,) * 3], [box], [r], 1.4, "outflow", 1e-3, 1e-3)
+    for lev, A in zip(H.levels, (U, Uf)):
+        lev.set_state(A)
+    dU = np.empty(U.shape)
+    hip.keep_null_stream_busy()
+    bsn.euler3d_rhs_(dU, None, None, None, g, *n, d, d, d, 1.4, bc="outflow")
+    H.step(2e-3)
+    np.testing.assert_array_equal(dU, O.euler3d_rhs(U.copy(), d, d, d, 1.4, "outflow", 0.0, 0.0)[0])
+    O.fmr_multilevel_step([U, Uf], [(d,) * 3, (d / r,) * 3], [box], [r], 1.4, 2e-3, "outflow", 1e-3, 1e-3)
+    for lev, A in zip(H.levels, (U, Uf)):
+        np.testing.assert_array_equal(lev.get_state(), A)
