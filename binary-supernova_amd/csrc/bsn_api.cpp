@@ -656,8 +656,7 @@ static int ensure_scratch(bsn_grid* g) { return ensure_buffer(g, g->d_scratch); 
 // reads its input with ghost cells mapped to active cells on load, and stage
 // 1 floors active cells on load, so no ghost fill or floor pass runs and A is
 // never modified before stage 3.
-static int plan_refresh(Plan& P) {
-    HIPCHK(hipSetDevice(P.ctx->device));
+static int plan_tables(Plan& P) {
     const auto G = host_descs(P);
     const size_t n = G.size();
     std::vector<GridDev> t(4 * n);
@@ -678,6 +677,20 @@ static int plan_refresh(Plan& P) {
     P.d_grids = P.desc.d;
     for (int s = 0; s < 3; ++s) P.d_st[s] = P.desc.d + (s + 1) * n;
     return BSN_OK;
+}
+
+// Every call on a batch or a hierarchy comes after what the null stream holds:
+// callers write states there (bsn_grid_device_state; torch's default stream is
+// the null stream), and the context's stream does not wait for it by itself.
+static int after_null_stream(bsn_ctx* c) {
+    HIPCHK(hipSetDevice(c->device));
+    HIPCHK(hipStreamSynchronize(nullptr));
+    return BSN_OK;
+}
+
+static int plan_refresh(Plan& P) {
+    CHK(after_null_stream(P.ctx));
+    return plan_tables(P);
 }
 
 static int plan_set_zshape(Plan& P, int shape) {
@@ -2280,13 +2293,14 @@ static int fmr_stage_tables(bsn_fmr* m, std::vector<GridDev>& t) {
 }
 
 static int fmr_refresh(bsn_fmr* m) {
+    CHK(after_null_stream(m->ctx));
     std::vector<GridDev> t;
     for (auto* g : m->lev) t.push_back(g->h);
     if (!m->inplace) CHK(fmr_stage_tables(m, t));
     CHK(m->all.set(m->ctx, t));
     m->d_all = m->all.d;
     m->d_fst = m->all.d + m->nlev;
-    for (auto* P : m->plans) CHK(plan_refresh(*P));
+    for (auto* P : m->plans) CHK(plan_tables(*P));
     return BSN_OK;
 }
 

@@ -116,3 +116,42 @@ def test_work_buffers_made_beside_a_busy_null_stream(hip):
     O.fmr_multilevel_step([U, Uf], [(d,) * 3, (d / r,) * 3], [box], [r], 1.4, 2e-3, "outflow", 1e-3, 1e-3)
     for lev, A in zip(H.levels, (U, Uf)):
         np.testing.assert_array_equal(lev.get_state(), A)
+
+
+def device_state(g):
+    p, fs = C.c_void_p(), C.c_int64()
+    call("bsn_grid_device_state", g.handle, C.byref(p), C.byref(fs), None)
+    return p, 5 * fs.value * 8
+
+
+@pytest.mark.parametrize("graph", [False, True])
+def test_states_written_on_the_null_stream(hip, graph):
+    # a new state reaches the grid's own buffer late, in the null stream's order,
+    # before each call on the batch and on the hierarchy
+    print(f"device states graph {graph}", flush=True)
+    n, nf, box, d = (18, 16, 20), (16, 16, 12), (6, 13, 5, 12, 8, 13), 0.1
+    news = [bsn.Grid(*s).set_state(state(s, 5 + k)) for k, s in enumerate((n, nf))]
+
+    def make():
+        g = bsn.Grid(*n).set_state(state(n, 7))
+        g.set_params(d, d, d, 1.4)
+        H = bsn.FMRHierarchy([n, nf], [(d,) * 3, (d / 2,) * 3], [box], [2], 1.4, "outflow", 1e-3, 1e-3)
+        for lev, s in zip(H.levels, (n, nf)):
+            lev.set_state(state(s, 8))
+        return g, bsn.Batch([g]), H
+
+    g, b, H = make()
+    for what, grids in ((b, [g]), (H, H.levels)):
+        for _ in range(2):                  # the first call, and one on kept tables
+            hip.keep_null_stream_busy()
+            for to, new in zip(grids, news):
+                (p, size), (q, _) = device_state(to), device_state(new)
+                hip.hipMemcpyAsync(p, q, size, D2D, None)
+            what.run(0.3, 2, graph=graph)
+    g2, b2, H2 = make()
+    for what, grids in ((b2, [g2]), (H2, H2.levels)):
+        for to, new in zip(grids, news):
+            to.set_state(new.get_state())
+        what.run(0.3, 2, graph=graph)
+    for x, y in zip([g] + H.levels, [g2] + H2.levels):
+        np.testing.assert_array_equal(x.get_state(), y.get_state())
