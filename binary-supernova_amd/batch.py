@@ -44,11 +44,13 @@ class Batch:
         segmentation: variant 0 plain, 1 operands loaded one cell ahead (FP64)
         or variant 3 without a register cap (split), 2 LDS ring of the
         window's raw cells, 3 ring + early window load; segmentation 0/1 = z
-        runs of 16/32 cells, 2 = balanced run lengths."""
+        runs of 16/32 cells, 2 = balanced run lengths.  12: the merged form of
+        small batches (three sweeps in one launch, then the update)."""
         call("bsn_batch_set_update_shape", self.handle, int(shape))
 
     def get_shapes(self) -> list:
-        """[x, y, z flux shape, fused-kernel shape] ids in use."""
+        """[x, y, z flux shape, fused-kernel shape] ids in use, the last 12
+        where steps take the merged form."""
         out = (C.c_int * 4)()
         call("bsn_batch_get_shapes", self.handle, out)
         return list(out)
@@ -74,7 +76,8 @@ class Batch:
     def profile(self, nsteps: int):
         """Runs nsteps device-dt steps with HIP events around every flux and
         update launch; returns (ms per flux launch [x, y, z], ms per update
-        launch, ms per step)."""
+        launch, ms per step).  Where steps take the merged form the profiled
+        ones run the separate kernels."""
         f3 = (C.c_double * 3)()
         u, s = C.c_double(), C.c_double()
         call("bsn_batch_profile", self.handle, int(nsteps), f3, C.byref(u), C.byref(s))

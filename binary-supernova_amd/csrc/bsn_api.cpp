@@ -276,7 +276,8 @@ struct Plan {
     int nft[3] = {0, 0, 0};
     Tile* d_ut = nullptr;
     // small grids (plan_small): one list for the three sweeps, one of single-cell
-    // update tiles; shapes set by the caller go back to the separate kernels
+    // update tiles.  small: steps take them (the merged form); shapes set by the
+    // caller go back to the separate kernels
     bool small = false;
     Tile* d_sw = nullptr;
     int nsw[3] = {0, 0, 0};
@@ -714,13 +715,14 @@ static int plan_set_zshape(Plan& P, int shape) {
 // tiles per CU the starts and the z fluxes' way through memory cost more than
 // the launches: at 5 per CU (56^3 has 4.4 to 4.7, 64^3 5.9) merged still wins.
 static const int SMALL_TILES = 5;
+static const int SMALL_SHAPE[3] = {0, FLUX_WALK_SHAPE0 + 2, FLUX_WALK_SHAPE0 + 2};
 static int plan_small(Plan& P, const std::vector<GridDev>& G) {
     const int64_t most = (int64_t)SMALL_TILES * P.ctx->cus;
     P.small = false;
     if (P.atotal > 256 * most) return BSN_OK;       // more x interfaces alone
     std::vector<Tile> t;
     for (int d = 0; d < 3; ++d) {
-        const auto l = flux_tiles(G, d, d == 0 ? 0 : FLUX_WALK_SHAPE0 + 2, P.ctx->cus, P.ctx->cus);
+        const auto l = flux_tiles(G, d, SMALL_SHAPE[d], P.ctx->cus, P.ctx->cus);
         P.nsw[d] = (int)l.size();
         t.insert(t.end(), l.begin(), l.end());
     }
@@ -732,6 +734,11 @@ static int plan_small(Plan& P, const std::vector<GridDev>& G) {
     P.small = true;
     return BSN_OK;
 }
+
+// The merged form's id beside those of the fused kernel's shapes, which it
+// stands in for; its lists exist where plan_small made them.
+static int merged_shape() { return zupdate_shape_count(); }
+static bool has_merged(const Plan& P) { return P.nut1 > 0; }
 
 static int plan_build(Plan& P) {
     HIPCHK(hipSetDevice(P.ctx->device));
@@ -1851,17 +1858,25 @@ extern "C" int bsn_batch_set_shapes(bsn_batch* b, int sx, int sy, int sz) {
 
 extern "C" int bsn_batch_set_update_shape(bsn_batch* b, int shape) {
     if (!b) return set_err(BSN_ERR_ARG, "NULL batch");
-    if (shape < 0 || shape >= zupdate_shape_count()) return set_err(BSN_ERR_ARG, "shape %d", shape);
-    HIPCHK(hipSetDevice(b->plan->ctx->device));
-    CHK(plan_set_zshape(*b->plan, shape));
-    b->plan->small = false;
+    Plan& P = *b->plan;
+    if (shape < 0 || shape > merged_shape()) return set_err(BSN_ERR_ARG, "shape %d", shape);
+    HIPCHK(hipSetDevice(P.ctx->device));
+    if (shape == merged_shape()) {
+        if (!has_merged(P)) return set_err(BSN_ERR_ARG, "shape %d: the merged form is for small batches", shape);
+        P.small = true;
+        graph_drop(P.gexec, P.graph);
+        return BSN_OK;
+    }
+    CHK(plan_set_zshape(P, shape));
+    P.small = false;
     return BSN_OK;
 }
 
 extern "C" int bsn_batch_get_shapes(bsn_batch* b, int shapes[4]) {
     if (!b || !shapes) return set_err(BSN_ERR_ARG, "NULL argument");
-    for (int d = 0; d < 3; ++d) shapes[d] = b->plan->shape[d];
-    shapes[3] = b->plan->zshape;
+    const Plan& P = *b->plan;
+    for (int d = 0; d < 3; ++d) shapes[d] = P.small ? SMALL_SHAPE[d] : P.shape[d];
+    shapes[3] = P.small ? merged_shape() : P.zshape;
     return BSN_OK;
 }
 
@@ -1872,8 +1887,6 @@ extern "C" int bsn_batch_set_mode(bsn_batch* b, int inplace) {
     return BSN_OK;
 }
 
-// Times every tile shape of every kernel of a plan on its current states and
-// keeps the fastest; appends a JSON object of the timings to rep.
 // Name of a flux-sweep shape in the autotuner's report: "WxH" for a tiled
 // shape, "walkL" for a register walk of L interfaces.
 static std::string flux_shape_name(int dir, int shape) {
@@ -1896,6 +1909,9 @@ static const char* zshape_name(int prec, int shape) {
     return names[prec == 1][shape];
 }
 
+// Times every tile shape of every kernel of a plan on its current states and
+// keeps the fastest, then, for small grids, the step of those kernels against
+// the merged form; appends a JSON object of the timings to out.
 static int plan_autotune(Plan& P, std::string& out) {
     HIPCHK(hipSetDevice(P.ctx->device));
     CHK(plan_refresh(P));
@@ -2006,6 +2022,35 @@ static int plan_autotune(Plan& P, std::string& out) {
     CHK(pick("zupdate", 3, zupdate_shape_count(),
              [&](int s) { return plan_set_zshape(P, s); },
              [&](int s) { return std::string(zshape_name(P.prec, s)); }));
+    // small grids: whole stages of the kept shapes against the merged form
+    if (has_merged(P)) {
+        auto stage_of = [&](bool merged, int stage) -> int {
+            if (!merged) return seq(-1, stage, nullptr);
+            HIPCHK(launch_sweeps(L, P.prec, P.d_st[stage - 1], P.d_sw, P.nsw));
+            HIPCHK(launch_update(L, P.prec, 1, P.d_st[stage - 1], P.d_ut1, P.nut1, stage, 0, nullptr));
+            return BSN_OK;
+        };
+        float t[2] = {1e30f, 1e30f};
+        for (int r = 0; r < passes; ++r)
+            for (int m = 0; m < 2; ++m) {
+                const int n = 10;
+                float ms = 0;
+                for (int q = 0; q < 2; ++q) CHK(stage_of(m, 1 + q));
+                HIPCHK(hipEventRecord(ev[0], L.stream));
+                for (int q = 0; q < 3 * n; ++q) CHK(stage_of(m, q % 3 == 0 ? 1 : 2));
+                HIPCHK(hipEventRecord(ev[1], L.stream));
+                HIPCHK(hipEventSynchronize(ev[1]));
+                HIPCHK(hipEventElapsedTime(&ms, ev[0], ev[1]));
+                t[m] = std::min(t[m], ms / (3 * n));
+            }
+        P.small = t[1] < t[0];
+        char buf[160];
+        snprintf(buf, sizeof buf, ", \"stage\": %.4f, \"merged_stage\": %.4f, \"merged\": %s}", t[0], t[1],
+                 P.small ? "true" : "false");
+        rep.pop_back();
+        rep += buf;
+        graph_drop(P.gexec, P.graph);
+    }
     rep += "}";
     HIPCHK(hipStreamSynchronize(L.stream));
     for (auto e : ev) (void)hipEventDestroy(e);

@@ -235,12 +235,17 @@ int bsn_batch_destroy(bsn_batch* b);
 /* Times every tile shape of every kernel on the current states and keeps the
  * fastest; writes a JSON report of the choice into report (may be NULL).
  * Without it a batch (and every FMR level and single-grid call) starts from
- * x 0, y/z 7 and fused kernel 11. */
+ * x 0, y/z 7 and fused kernel 11, or, where its grids are small (56^3 in all
+ * and less, about), from the merged form: the three sweeps in one launch, then
+ * an update of one cell per thread.  For such a batch the tuner also times a
+ * stage of the kernels it kept ("stage", ms) against one of the merged form
+ * ("merged_stage") and keeps the faster ("merged"). */
 int bsn_batch_autotune(bsn_batch* b, char* report, int report_len);
 /* Sets the flux shape ids explicitly (x: 0..2 tiled, 3..5 walks of 2, 4 and 4
  * interfaces per lane through LDS-staged rows, the last storing its fluxes
  * directly; y/z: 0..4 tiled, 5..7
- * register walks along the sweep of 16, 32 or 64 interfaces per thread). */
+ * register walks along the sweep of 16, 32 or 64 interfaces per thread).
+ * Steps then take the separate kernels, also where the grids are small. */
 int bsn_batch_set_shapes(bsn_batch* b, int sx, int sy, int sz);
 /* Sets the shape id (0..11) of the fused z-sweep + stage-update kernel used
  * by the out-of-place step: shape = 3 * variant + segmentation.  Variant 0
@@ -248,10 +253,12 @@ int bsn_batch_set_shapes(bsn_batch* b, int sx, int sy, int sz);
  * the window's raw cells in an LDS ring instead of reading them twice, 3 the
  * ring plus an early load of the next window cell.  Segmentation 0 and 1: z
  * runs of 16 or 32 cells per column tile; 2: one run length per grid chosen
- * so that the tiles fill the resident workgroups evenly. */
+ * so that the tiles fill the resident workgroups evenly.  Shape 12: the merged
+ * form, for batches of small grids only (BSN_ERR_ARG otherwise). */
 int bsn_batch_set_update_shape(bsn_batch* b, int shape);
 /* The shape ids in use: x, y, z flux shapes and the fused kernel's shape (as
- * the autotuner left them), for bsn_batch_set_shapes / _set_update_shape. */
+ * the autotuner left them; 12 where steps take the merged form), for
+ * bsn_batch_set_shapes and then bsn_batch_set_update_shape. */
 int bsn_batch_get_shapes(bsn_batch* b, int shapes[4]);
 /* Step form: 0 (default) = out of place, z sweep fused with the stage update;
  * 1 = in place with all fluxes materialised.  Both give the same bits. */
@@ -322,8 +329,9 @@ int bsn_fmr_restrict_density(bsn_fmr* m, int level);
 int bsn_fmr_prolong_scalar(bsn_fmr* m, int level, const double* phi_c, int where_c,
                            double* phi_f, int where_f);
 
-/* Kernel timing of the last bsn_batch_run / bsn_fmr_run with profile=1:
- * average milliseconds per launch of the flux (x, y, z) and update kernels. */
+/* nsteps device-dt steps with events around the kernels: average milliseconds
+ * per launch of the flux (x, y, z) and update kernels, and per step.  Where
+ * steps take the merged form the profiled ones run the separate kernels. */
 int bsn_batch_profile(bsn_batch* b, int nsteps, double* ms_flux3, double* ms_update,
                       double* ms_step);
 
