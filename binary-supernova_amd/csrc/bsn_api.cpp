@@ -84,17 +84,24 @@ struct bsn_ctx {
     LaunchCtx L() const { return LaunchCtx{stream, cus}; }
 };
 
-// Copies between host arrays and the device on the context's stream, a slot of
-// pinned memory at a time: the CPU fills or empties one while the others are in
-// flight.  The link moves 13.7 MB in 250 us and 256 kB in 13; left to the runtime,
-// pageable memory takes 800 us to the host, and 110 for the 256 kB either way.  Here
-// one thread's copying (28 GB/s from memory, 62 to it) sets the pace: a host loop
-// on numpy arrays takes 0.19 ms per step at 8^3 (0.50 by the runtime's copies), 0.60
-// at 32^3 (0.82), 2.1 at 64^3 (2.5).  Three helper threads doubled the copying, but
-// their start cost a 4 MB array more (40^3 1.43 ms against 0.93) than they gave a
-// 14 MB one.  Memory that is pinned already (or managed) is copied directly, and
-// the copy waited for: the caller may write to it, or free it, as soon as it has
-// it back.
+// Copies between host arrays and the device on the context's stream, by the
+// runtime or through slots of pinned memory, of which the CPU fills or empties
+// one while the others are in flight.  Times of whole calls, pageable arrays:
+//   in    the runtime, which takes set_state 24 us for 50 kB, 100 for 2 MB (through
+//         slots 28 and 107).
+//   post  up to 3 MB through slots: the caller goes on 6 us after it began (the
+//         runtime 14), 15 for 512 kB (38), and the kernels it launches follow.
+//   out   above 1 MB, where there is more than one part, through slots: get_state
+//         2 MB 110 us (the runtime 135), 14 MB 580 (800); one thread's copying
+//         sets the pace.  So do several arrays of one call: dU and three fluxes
+//         of 32^3 0.70 ms (1.00).  Below that the runtime: 50 kB 28 us (slots 34).
+//         Up to 16 kB a slot again, without an event: solve_poisson_isolated of
+//         8^3 32 us (the runtime 40, with an event 68).
+// A host loop on numpy arrays takes 0.17 ms per step at 8^3 (0.36 by the runtime's
+// copies alone), 0.47 at 32^3 (0.65), 1.8 at 64^3 (2.2).  Three helper threads
+// doubled the copying, but their start cost a 4 MB array more (40^3 1.43 ms against
+// 0.93) than they gave a 14 MB one.  Memory that is pinned already (or managed) is
+// copied directly.
 //
 // The object holds the pipe for as long as it lives; data has arrived in host
 // arrays after flush().
@@ -102,12 +109,10 @@ class HostXfer {
     bsn_ctx* c;
     std::lock_guard<std::mutex> lk;
     bool direct = false;     // a copy straight to the caller's memory is in flight
-    struct Out { char* dst; size_t n; int slot; } q[HostPipe::SLOTS];    // not taken yet, oldest first
+    struct Out { char* dst; size_t n; int slot; bool ev; } q[HostPipe::SLOTS];   // not taken yet, oldest first
     int qn = 0;
 
-    // the runtime's own copy from pageable memory is as fast beyond this (139 us for
-    // 4.2 MB; 367 for 1 MB, here 45)
-    static const size_t DIRECT_FROM = 3 << 20;
+    static const size_t POST_TO = 3 << 20, SMALL = 16 << 10;
 
     char* mem(int s) const { return c->pipe.buf + s * HostPipe::SLOT; }
     // a copy has its launch and its event to pay (14 us): parts of 1 MB, 2 of
@@ -125,7 +130,8 @@ class HostXfer {
     int take() {
         HostPipe& p = c->pipe;
         const Out o = q[0];
-        HIPCHK(hipEventSynchronize(p.ev[o.slot]));
+        if (o.ev) HIPCHK(hipEventSynchronize(p.ev[o.slot]));
+        else      HIPCHK(hipStreamSynchronize(c->stream));
         p.busy[o.slot] = false;
         memcpy(o.dst, mem(o.slot), o.n);
         for (int i = 1; i < qn; ++i) q[i - 1] = q[i];
@@ -163,12 +169,18 @@ public:
     HostXfer(const HostXfer&) = delete;
     HostXfer& operator=(const HostXfer&) = delete;
 
-    // on return src has been read
+    // for callers that wait for the stream later in the call (src may be read until
+    // then)
     int in(void* dst, const void* src, size_t n) {
+        HIPCHK(hipMemcpyAsync(dst, src, n, hipMemcpyHostToDevice, c->stream));
+        return BSN_OK;
+    }
+    // for those that do not: on return src has been read
+    int post(void* dst, const void* src, size_t n) {
         const bool paged = pageable(src);
-        if (n > DIRECT_FROM || !paged) {
+        if (n > POST_TO || !paged) {
             // from pageable memory the runtime's copy returns when it has read it
-            HIPCHK(hipMemcpyAsync(dst, src, n, hipMemcpyHostToDevice, c->stream));
+            CHK(in(dst, src, n));
             if (!paged) HIPCHK(hipStreamSynchronize(c->stream));
             return BSN_OK;
         }
@@ -183,8 +195,10 @@ public:
         }
         return BSN_OK;
     }
-    int out(void* dst, const void* src, size_t n) {
-        if (!pageable(dst)) {
+    // more: other arrays of the call follow
+    int out(void* dst, const void* src, size_t n, bool more = false) {
+        const bool one = qn == 0 && !more && n > SMALL && n <= part(n);
+        if (one || !pageable(dst)) {
             HIPCHK(hipMemcpyAsync(dst, src, n, hipMemcpyDeviceToHost, c->stream));
             direct = true;
             return BSN_OK;
@@ -195,8 +209,9 @@ public:
             int s;
             CHK(slot(s));
             HIPCHK(hipMemcpyAsync(mem(s), (const char*)src + o, k, hipMemcpyDeviceToHost, c->stream));
-            CHK(sent(s));
-            q[qn++] = {(char*)dst + o, k, s};
+            const bool ev = n > SMALL;
+            if (ev) CHK(sent(s));
+            q[qn++] = {(char*)dst + o, k, s, ev};
         }
         return BSN_OK;
     }
@@ -232,7 +247,7 @@ struct DescTable {
         }
         held.clear();
         HostXfer x(c);
-        CHK(x.in(d, v.data(), bytes));
+        CHK(x.post(d, v.data(), bytes));
         held = v;
         return BSN_OK;
     }
@@ -1154,7 +1169,7 @@ static int src_upload(bsn_grid* g) {
     if (any) {
         if (!g->d_src) HIPCHK(hipMalloc((void**)&g->d_src, sizeof(SrcDev)));
         HostXfer x(g->ctx);
-        CHK(x.in(g->d_src, &S, sizeof(SrcDev)));
+        CHK(x.post(g->d_src, &S, sizeof(SrcDev)));
     }
     const SrcDev* want = any ? g->d_src : nullptr;
     if (g->h.src != want) {
@@ -1300,7 +1315,12 @@ extern "C" int bsn_solve_poisson_isolated(bsn_grid* g, const double* rho, int wh
     HostXfer x(g->ctx);
     if (where_rho == BSN_HOST) CHK(x.in(g->d_rho_in, rho, n * 8));
     HIPCHK(poisson_solve_array(*g->pois, drho, dphi, g->ctx->stream));
-    if (where_phi == BSN_HOST) CHK(x.out(phi, dphi, n * 8));
+    if (where_phi == BSN_HOST) {
+        // the events of two to four parts cost more behind the transforms than on
+        // an idle stream: 64^3 269 us, 238 with the wait; 80^3 501 and 504
+        if (n * 8 > (1 << 20) && n * 8 <= (4 << 20)) CHK(sync_ctx(g->ctx));
+        CHK(x.out(phi, dphi, n * 8));
+    }
     CHK(x.flush());
     return sync_ctx(g->ctx);
 }
@@ -1341,7 +1361,7 @@ extern "C" int bsn_grid_set_phi(bsn_grid* g, const double* phi, int where) {
     if (!g->d_phi) HIPCHK(hipMalloc((void**)&g->d_phi, bytes));
     if (where == BSN_HOST) {
         HostXfer x(g->ctx);
-        CHK(x.in(g->d_phi, phi, bytes));
+        CHK(x.post(g->d_phi, phi, bytes));
     } else {
         // after what the null stream still has to write to phi; such a copy may be
         // on its way when hipMemcpy returns, and neither the caller's next write
@@ -1445,7 +1465,7 @@ extern "C" int bsn_euler3d_rhs(bsn_grid* g, double* dU, double* Fx, double* Fy, 
         if (where == BSN_HOST) {
             CHK(ensure_stage(g, n * 8));
             HIPCHK(launch_flux_export(L, h, d, g->d_stage));
-            CHK(x.out(F[d], g->d_stage, n * 8));
+            CHK(x.out(F[d], g->d_stage, n * 8, d < 2 || dU));
         } else {
             HIPCHK(launch_flux_export(L, h, d, F[d]));
         }
@@ -2580,7 +2600,7 @@ extern "C" int bsn_solve_fmr_poisson(bsn_fmr* m, double* const* phi, int where) 
     CHK(fmr_sg_solve(m, dst.data(), 1.0));
     HostXfer x(m->ctx);
     if (where == BSN_HOST)
-        for (int l = 0; l < m->nlev; ++l) CHK(x.out(phi[l], dst[l], active_cells(m->lev[l]->h) * 8));
+        for (int l = 0; l < m->nlev; ++l) CHK(x.out(phi[l], dst[l], active_cells(m->lev[l]->h) * 8, l + 1 < m->nlev));
     CHK(x.flush());
     return sync_ctx(m->ctx);
 }

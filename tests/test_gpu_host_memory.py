@@ -1,6 +1,7 @@
-"""GPU: calls on page-locked host arrays, which the library copies directly: what
-a call was given has been read, and what it returns has arrived, when it
-returns.  The oracle sees the values each call was given."""
+"""GPU: calls on host arrays, page-locked ones, which the library copies directly,
+and ordinary ones of sizes around which its copies change: what a call was given
+has been read, and what it returns has arrived, when it returns.  The oracle
+sees the values each call was given."""
 import ctypes as C
 
 import numpy as np
@@ -101,3 +102,34 @@ def test_states_through_pinned_arrays(pinned, shape):
     sg_force(g, dU)
     O.apply_sg_force(want, U, phi, *D)
     np.testing.assert_array_equal(dU, want)
+
+
+# bytes of a state around 16 kB (a small slot without an event), 1 MB (one part
+# or several) and 8 MB (parts of 1 or 2 MB)
+@pytest.mark.parametrize("nx", [1, 2, 3, 528, 529, 4273, 4274])
+def test_states_of_every_transfer_size(nx):
+    print(f"state transfers {nx}", flush=True)
+    U = np.random.default_rng(nx).normal(size=(7, 7, nx + 6, 5))
+    g = bsn.Grid(nx, 1, 1)
+    for k in range(3):
+        g.set_state(U + k)
+        np.testing.assert_array_equal(g.get_state(), U + k)
+
+
+# up to 3 MB posted through slots, more of them than there are, or straight
+@pytest.mark.parametrize("nz", [96, 97])
+def test_phis_posted_one_after_the_other(nz):
+    print(f"posted phis {nz}", flush=True)
+    shape = (64, 64, nz)
+    U = state(shape, 5)
+    grids = [bsn.Grid(*shape).set_state(U) for _ in range(3)]
+    phi = np.empty(shape[::-1])
+    for k, g in enumerate(grids):
+        phi[...] = 0.1 * np.random.default_rng(k).normal(size=phi.shape)
+        g.set_phi(phi)
+        phi[...] = 7.0
+    for k, g in enumerate(grids):
+        dU, want = np.zeros(U.shape), np.zeros(U.shape)
+        sg_force(g, dU)
+        O.apply_sg_force(want, U, 0.1 * np.random.default_rng(k).normal(size=phi.shape), *D)
+        np.testing.assert_array_equal(dU, want)
