@@ -931,10 +931,16 @@ static int plan_step_inplace(Plan& P, int device_dt) {
     return BSN_OK;
 }
 
+// The maximum of small grids takes the single-cell tiles while their atomics, one
+// per tile, cost less than the columns' serial loads: cfl_dt_3d of 32^3 (256
+// tiles) 22 us against 25 with columns, 48^3 (576) 25.7 and 26.3, 52^3 (676) 27.0
+// and 26.4, 17 x 130 x 70 (2310) 46 and 29.
+static const int CFL1_TILES = 600;
+
 static int plan_cfl(Plan& P, double cfl, double t_end, int restart = 0) {
     const LaunchCtx L = P.ctx->L();
     HIPCHK(launch_cfl_begin(L, P.d_grids, (int)P.grids.size(), cfl, t_end, restart));
-    if (P.small) HIPCHK(launch_cfl(L, 1, P.d_grids, P.d_ut1, P.nut1));
+    if (P.small && P.nut1 <= CFL1_TILES) HIPCHK(launch_cfl(L, 1, P.d_grids, P.d_ut1, P.nut1));
     else         HIPCHK(launch_cfl(L, UPDATE_KZ, P.d_grids, P.d_ut, P.nut));
     return BSN_OK;
 }
