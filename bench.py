@@ -112,6 +112,7 @@ def run_uniform(bsn, U, dims, d, gamma, bc, floors, prec, steps, warmup, cfl=0.4
     if warmup:
         b.run(cfl, warmup, graph=True)
         g.set_state(U)
+    b.run(cfl, 0)           # the first step's dt: the CFL number and this state's maximum
     g.ctx.synchronize()
     t0 = time.perf_counter()
     ms_flux, ms_upd, ms_step = b.profile(steps)
@@ -545,6 +546,7 @@ def bench_selfgrav(bsn, args):
         bsn.set_self_gravity(g, True)
         b.run(0.4, args.warmup, graph=False)
         g.set_state(U)
+        b.run(0.4, 0)       # the first step's dt
         g.ctx.synchronize()
         t0 = time.perf_counter()
         ms_flux, ms_upd, ms_step = b.profile(steps)

@@ -76,8 +76,9 @@ class Batch:
     def profile(self, nsteps: int):
         """Runs nsteps device-dt steps with HIP events around every flux and
         update launch; returns (ms per flux launch [x, y, z], ms per update
-        launch, ms per step).  Where steps take the merged form the profiled
-        ones run the separate kernels."""
+        launch, ms per step).  The first dt is of the CFL number and maximum
+        that run() left: after new states call run(cfl, 0) first.  Where steps
+        take the merged form the profiled ones run the separate kernels."""
         f3 = (C.c_double * 3)()
         u, s = C.c_double(), C.c_double()
         call("bsn_batch_profile", self.handle, int(nsteps), f3, C.byref(u), C.byref(s))

@@ -330,8 +330,10 @@ int bsn_fmr_prolong_scalar(bsn_fmr* m, int level, const double* phi_c, int where
                            double* phi_f, int where_f);
 
 /* nsteps device-dt steps with events around the kernels: average milliseconds
- * per launch of the flux (x, y, z) and update kernels, and per step.  Where
- * steps take the merged form the profiled ones run the separate kernels. */
+ * per launch of the flux (x, y, z) and update kernels, and per step.  It goes
+ * on from the CFL number and the wave-speed maximum that bsn_batch_run left
+ * (after new states call that with nsteps = 0 first; without it dt is Inf).
+ * Where steps take the merged form the profiled ones run the separate kernels. */
 int bsn_batch_profile(bsn_batch* b, int nsteps, double* ms_flux3, double* ms_update,
                       double* ms_step);
 
