@@ -455,9 +455,11 @@ static void balance_chunks(std::vector<Tile>& t, int slots, Weight weight) {
 // its start) and takes at most lmax.  A workgroup's waves share their CU's
 // SIMDs with those of the other resident workgroups, so what matters is the
 // largest sum of runs on a CU; a CU that holds w workgroups where occ fit works
-// at lone + (1 - lone) w / occ of its rate.  The split kernels wait on memory
-// and need their waves more: lone 0.2 gave 64^3 0.378 ms for two steps, 0.4
-// 0.401; FP64 0.4 0.601 ms, 0.75 0.622.
+// at lone + (1 - lone) w / occ of its rate.  The split kernels wait on memory and
+// need their waves more.  Of lone 0.1, 0.2, 0.4, 0.75 and 1 on 13 single grids from
+// 60^3 to 192^3, 0.2 is within 1.4 % of the best for split steps (but 60^3, 2.4 %)
+// and 0.4 within 0.7 % for FP64 (but 97 x 61 x 45, 1.7 %): split 64^3 149 us per step,
+// 157 with 0.4, 162 with 1; FP64 80^3 389 us, 388 with 0.1, 418 with 1.
 //
 // One grid: the count s of runs per column that minimises that sum over
 // cols * s equal runs, down to runs of 1 where the grid is too small to fill
@@ -466,7 +468,10 @@ static void balance_chunks(std::vector<Tile>& t, int slots, Weight weight) {
 // gave a 192^3 grid 576 runs, 2.25 per CU, with the double chunks on one XCD:
 // its FP64 step took 5.41 ms against 4.00.)
 // Several grids: one length for all, from a few candidates, by the mean load
-// of a CU plus half a run for the uneven end.
+// of a CU plus half a run for the uneven end.  Seven batches of 3 to 48 grids in
+// both forms took 0.98 of the time they take with one length that fills the
+// resident workgroups a whole number of times (0.88 to 1.08 each), 0.99 without
+// the half run.
 static std::vector<int> run_counts(const std::vector<int>& cols, const std::vector<int>& len, double c,
                                    double lmax, int cus, int occ, int prec) {
     const size_t N = cols.size();
@@ -2467,8 +2472,8 @@ extern "C" int bsn_fmr_set_mode(bsn_fmr* m, int inplace) {
 }
 
 // Each level's plan tuned on the level's current state (the timing launches
-// write the level's flux arrays and its Un buffer, which every level step
-// rebuilds before reading).
+// write the level's flux arrays and its Un buffer, of which every level step
+// rebuilds what it reads).
 extern "C" int bsn_fmr_autotune(bsn_fmr* m, char* report, int report_len) {
     if (!m) return set_err(BSN_ERR_ARG, "NULL fmr");
     HIPCHK(hipSetDevice(m->ctx->device));

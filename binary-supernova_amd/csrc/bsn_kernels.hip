@@ -2304,9 +2304,9 @@ static int zupdate_slots_t(int cus) {
 // Shapes: 3 * variant + segmentation.  Variant 0 plain, 1 operands loaded one
 // cell ahead (FP64) or variant 3 without a register cap (split: 2 waves per
 // SIMD), 2 LDS ring of the window's raw cells, 3 ring plus an early load of
-// the next window cell (split: both capped at 168 VGPRs, 3 waves per SIMD).  Segmentation 0: 16 cells per column tile, 1: 32,
-// 2: one length per grid chosen so the tile count fills the resident
-// workgroup slots (zupdate_slots) evenly.
+// the next window cell (split: both capped at 168 VGPRs, 3 waves per SIMD).
+// Segmentation 0: at most 16 cells per run, 1: 32, 2: runs balanced by the load of
+// a CU (run_counts in bsn_api.cpp).
 int zupdate_shape_count() { return 12; }
 int zupdate_seg(int shape) { return shape % 3; }
 

@@ -259,9 +259,10 @@ __device__ __forceinline__ void interface_flux_plain(At&& at, double g, double g
 // are those of the full division.  WENO5-Z has 12 divisions per quantity by 7
 // distinct denominators; a walk carries the reciprocals of the indicators
 // that consecutive interfaces share, which leaves 5.  HLLC divides 7 times by
-// each side's density.  At 256^3 an FP64 y walk issues 1268 VALU instructions
-// per interface instead of 1949: 1.13 -> 0.79 ms; the tiled x sweep 1.18 ->
-// 0.89 ms, the fused z sweep and update 1.38 -> 1.12 ms, the step 11.4 -> 8.75.
+// each side's density.  At 256^3 an FP64 y walk issues 1259 VALU instructions
+// per interface instead of 1948: 1.16 -> 0.79 ms; the tiled x sweep 1998 -> 1440,
+// 1.21 -> 0.91 ms, the fused z sweep and update 2129 -> 1537, 1.40 -> 1.15 ms, the
+// step 11.4 -> 8.7.
 //
 // Ranges.  interface_flux_shared refuses (the callers then take
 // interface_flux_plain) unless every rho of the stencil is below 2^96 in

@@ -252,8 +252,8 @@ int bsn_batch_set_shapes(bsn_batch* b, int sx, int sy, int sz);
  * plain, 1 loads the next cell and the update operands one cell ahead, 2 keeps
  * the window's raw cells in an LDS ring instead of reading them twice, 3 the
  * ring plus an early load of the next window cell.  Segmentation 0 and 1: z
- * runs of 16 or 32 cells per column tile; 2: one run length per grid chosen
- * so that the tiles fill the resident workgroups evenly.  Shape 12: the merged
+ * runs of 16 or 32 cells per column tile; 2: runs balanced by the load of a
+ * CU, at most 96 cells.  Shape 12: the merged
  * form, for batches of small grids only (BSN_ERR_ARG otherwise). */
 int bsn_batch_set_update_shape(bsn_batch* b, int shape);
 /* The shape ids in use: x, y, z flux shapes and the fused kernel's shape (as
