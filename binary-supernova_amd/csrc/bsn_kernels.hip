@@ -836,7 +836,7 @@ __global__ __launch_bounds__(256) void k_fxwalk(const GridDev* __restrict__ grid
 // cell per interface straight from HBM (lanes along x: coalesced), and the
 // split form carries the smoothness indicators that consecutive interfaces
 // share.  A run of len interfaces reads len + 5 cells.
-// The FP64 form carries them too, with their reciprocals, at 255 VGPRs, 2 waves
+// The FP64 form carries them too, with their reciprocals, at 252 VGPRs, 2 waves
 // per SIMD.
 template <int DIR, typename T>
 __device__ __forceinline__ void walk_tiles(const GridDev* __restrict__ grids, const Tile* __restrict__ tiles,
